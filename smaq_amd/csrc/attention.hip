@@ -447,6 +447,9 @@ struct Plan {
   int64_t hist_split, recent_split;
   int s_hist, s_recent;
   bool mfma, prefill;
+  // matrix-core row kernel for the history (s_hist is then 0: its partials
+  // have a layout of their own)
+  bool rows;
   // matrix-core decode with one workgroup per (sequence, KV head) and
   // per-sequence lengths: dispatch the longest sequences first
   bool longest_first;
@@ -472,13 +475,20 @@ constexpr int kDecodeMaxPieces = 8;
 
 static int64_t align256(int64_t x) { return (x + 255) & ~(int64_t)255; }
 
-static Plan make_plan(const smaq_attn_params* p) {
+static Plan make_plan(const smaq_attn_params* p, bool allow_rows) {
   Plan pl;
   const int g = p->n_q_heads / p->n_kv_heads;
   const int rows = p->q_len * g;
   pl.row_tiles = (rows + kRowTile - 1) / kRowTile;
   pl.mfma = (p->impl == 0 || p->impl == 2) && p->has_history && mfma_decode_supported(*p);
   pl.prefill = (p->impl == 0 || p->impl == 3) && !pl.mfma && prefill_mfma_supported(*p);
+  // The row kernel merges the recent window's partials, so that phase has to
+  // be in the same call.  It wins wherever it is supported: 37x at 16 x 32768
+  // tokens, 43x at 64 paged sequences (attention_rows.h), 2.9x for the whole
+  // call at 5 query tokens over 4001, 3x at 16 tokens.
+  const int phase_mask = p->phases ? p->phases : 15;
+  pl.rows = allow_rows && !pl.mfma && !pl.prefill && rows_supported(*p) &&
+            (!p->has_recent || p->max_recent_len <= 0 || (phase_mask & 3) == 3);
   const int64_t units = (int64_t)p->batch * p->n_kv_heads * pl.row_tiles;
   // aim for >= 2048 workgroups over the history
   int64_t want = units >= 2048 ? 1 : (2048 + units - 1) / units;
@@ -497,7 +507,7 @@ static Plan make_plan(const smaq_attn_params* p) {
     pl.hist_lp = prefill_padded_len(hl);
     pl.recent_lp = prefill_padded_len(rl);
   }
-  pl.s_hist = hl > 0 ? (int)((hl + pl.hist_split - 1) / pl.hist_split) : 0;
+  pl.s_hist = hl > 0 && !pl.rows ? (int)((hl + pl.hist_split - 1) / pl.hist_split) : 0;
   pl.s_recent = rl > 0 ? (int)((rl + pl.recent_split - 1) / pl.recent_split) : 0;
   // With ragged lengths and a single split per sequence the workgroups differ
   // in length by up to max / min; dispatched in batch order, the long ones
@@ -547,10 +557,10 @@ static int64_t partial_bytes(const smaq_attn_params* p, const Plan& pl) {
 
 using namespace smaq;
 
-extern "C" long long smaq_attn_workspace_bytes(const smaq_attn_params* p) {
-  if (!p || p->n_kv_heads <= 0 || p->n_q_heads % p->n_kv_heads) return -1;
-  const Plan pl = make_plan(p);
+// Workspace of a call that runs as `pl`.
+static int64_t plan_bytes(const smaq_attn_params* p, const Plan& pl) {
   int64_t bytes = partial_bytes(p, pl);
+  if (pl.rows) return align256(bytes) + rows_bytes(*p);
   if (pl.longest_first) bytes = align256(bytes) + order_bytes(p, pl);
   if (pl.prefill) {
     // tile images, value-lo planes and tile errors of each part
@@ -558,6 +568,18 @@ extern "C" long long smaq_attn_workspace_bytes(const smaq_attn_params* p) {
             prefill_planes_bytes(p->batch, p->n_kv_heads, pl.recent_lp);
   }
   return bytes;
+}
+
+// Whatever the phases of the calls that share the workspace: enough for the
+// generic kernels, and for the row kernel unless that alone would pass the
+// built-in scratch's size.
+extern "C" long long smaq_attn_workspace_bytes(const smaq_attn_params* p) {
+  if (!p || p->n_kv_heads <= 0 || p->n_q_heads % p->n_kv_heads) return -1;
+  const int64_t bytes = plan_bytes(p, make_plan(p, false));
+  const Plan rows = make_plan(p, true);
+  if (!rows.rows) return bytes;
+  const int64_t more = plan_bytes(p, rows);
+  return more <= bytes || (more > SMAQ_NOALLOC_SCRATCH_BYTES && bytes <= SMAQ_NOALLOC_SCRATCH_BYTES) ? bytes : more;
 }
 
 template <int KEY, typename TN, typename TV>
@@ -613,7 +635,10 @@ extern "C" int smaq_attn_hybrid(const smaq_attn_params* pp, void* stream) {
     SMAQ_REQUIRE((p.q_exact || p.q_raw) && p.recent_k && p.recent_v && p.max_recent_len > 0,
                  "smaq_attn_hybrid: null recent pointer");
   }
-  const Plan pl = make_plan(&p);
+  Plan pl = make_plan(&p, true);
+  // (a caller that sized its workspace before it set the arrival counters
+  // has room for the generic kernels only)
+  if (pl.rows && plan_bytes(&p, pl) > p.workspace_bytes) pl = make_plan(&p, false);
   if (p.impl == 2 && !pl.mfma) {
     set_error("smaq_attn_hybrid: the matrix-core decode kernel does not serve this shape");
     return SMAQ_EUNSUPPORTED;
@@ -623,7 +648,7 @@ extern "C" int smaq_attn_hybrid(const smaq_attn_params* pp, void* stream) {
     return SMAQ_EUNSUPPORTED;
   }
   SMAQ_REQUIRE(p.impl >= 0 && p.impl <= 3, "smaq_attn_hybrid: unknown impl %d", p.impl);
-  const long long need = smaq_attn_workspace_bytes(&p);
+  const long long need = plan_bytes(&p, pl);
   SMAQ_REQUIRE(p.workspace_bytes >= need, "smaq_attn_hybrid: workspace %lld < %lld bytes",
                p.workspace_bytes, need);
   const int S = pl.s_hist + pl.s_recent;
@@ -658,7 +683,7 @@ extern "C" int smaq_attn_hybrid(const smaq_attn_params* pp, void* stream) {
     }
     return launch_status("smaq_attn_hybrid(recent)");
   };
-  const bool recent_first = merge && pl.s_recent > 0;
+  const bool recent_first = (merge || pl.rows) && pl.s_recent > 0;
   // The query rotation (given rot_mt) is one launch into q_hist ahead of
   // the history phase (phase 8); when the recent window goes first as well
   // (and has the decode kernel), one launch runs both side by side.
@@ -725,6 +750,11 @@ extern "C" int smaq_attn_hybrid(const smaq_attn_params* pp, void* stream) {
                            p.recent_pos_offset, pl.s_hist};
       if ((rc = launch_prefill_mfma(p, pp, pl.s_recent, part, st)) != SMAQ_OK) return rc;
     }
+  } else if (pl.rows && (phases & 1)) {
+    const HistAddr a{p.hist_seq_start, p.max_hist_len, p.hist_head_stride, p.block_table, p.max_blocks,
+                     p.block_size, p.n_kv_heads};
+    const int rc = launch_rows(p, a, (char*)p.workspace + align256(partial_bytes(&p, pl)), part, pl.s_recent, st);
+    if (rc != SMAQ_OK) return rc;
   } else if (pl.s_hist > 0 && (phases & 1)) {
     HistAddr a{p.hist_seq_start, p.max_hist_len, p.hist_head_stride, p.block_table, p.max_blocks,
                p.block_size, p.n_kv_heads};
@@ -757,7 +787,7 @@ extern "C" int smaq_attn_hybrid(const smaq_attn_params* pp, void* stream) {
     const int rc = launch_recent();
     if (rc != SMAQ_OK) return rc;
   }
-  if (!(phases & 4) || direct || merge) return SMAQ_OK;
+  if (!(phases & 4) || direct || merge || pl.rows) return SMAQ_OK;
   dim3 cgrid((unsigned)((rows + kCombineRows - 1) / kCombineRows), p.n_kv_heads, p.batch);
   const dim3 cblock((unsigned)((p.head_dim + 63) / 64 * 64), kCombineRows);  // one thread per output dim
   switch (p.out_dtype) {

@@ -1,0 +1,132 @@
+"""The matrix-core row kernel (attention_rows.h: block-VQ keys, more than 4
+query rows per KV head, 4-bit values) against the generic kernels (impl 1,
+oracle-checked in test_gpu_attention.py), at its tile and share edges.
+
+Outputs are fp32.  Either side's logits are within 2^-22 * sum |q k| * scale of
+the exact ones (at most 40 here: 1e-5), its weights within as much relative,
+and the weights sum to 1, so outputs agree to 2e-5 * max |v|."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import smaq_amd as S
+from smaq_amd.batch import PagedQuantizedKV, QuantizedKVBatch
+from tests.conftest import sample_keys
+
+pytestmark = pytest.mark.gpu
+
+
+def _strategy(dev, codec, size, seed=0):
+    if codec == "scalar":
+        return S.SMAQFullMetricScalarStrategy(128, bits=size, device=dev).fit(sample_keys(64, seed=seed + 5))
+    nc = 100 if size == 4 else 256
+    strat = S.SMAQBlockVQStrategy(128, block_dim=size, n_centroids=nc, device=dev)
+    x = sample_keys(nc, seed=seed + 6).reshape(nc, 128 // size, size).transpose(0, 1).contiguous().to(dev)
+    strat.quantizer.load_state_dict({**strat.quantizer.state_dict(), "centroids": x, "decoded_centroids": x})
+    return strat
+
+
+def _close(got, ref, vals, what):
+    diff = float((got - ref).abs().max())
+    print(f"\n[{what}] max|err| {diff:.2e}")
+    assert diff <= 2e-5 * float(max(v.float().abs().max() for v in vals)), what
+
+
+# (codec, key bits or block dim, value bits, heads per KV head, query tokens, storage dtype)
+FORMS = [("vq", 2, 2, 7, 1, torch.float16), ("vq", 4, 4, 8, 1, torch.bfloat16), ("vq", 8, 2, 4, 3, torch.bfloat16),
+         ("vq", 8, 4, 1, 1, torch.float32), ("scalar", 3, 2, 7, 1, torch.bfloat16), ("scalar", 4, 4, 3, 1, torch.float16),
+         ("scalar", 3, 4, 2, 15, torch.float32), ("scalar", 4, 2, 16, 2, torch.float32)]
+
+
+@pytest.mark.parametrize("codec,size,vbits,g,T,dtype", FORMS)
+def test_rows_store_edges(dev, codec, size, vbits, g, T, dtype):
+    """One sequence, lengths around the 32-token tile, the steps of 128 and 256
+    tokens and a share of several steps; with and without a recent window and
+    a causal limit; a repeated call gives the same bits."""
+    strat = _strategy(dev, codec, size)
+    for n, rn in ((16, 0), (33, 1), (127, 64), (257, 65), (513, 0), (2051, 128)):
+        st = S.CompressedKVStore(128, 2, value_bits=vbits, device=dev, key_strategy=strat)
+        k = sample_keys(n * 2, seed=n).view(n, 2, 128).to(dtype).to(dev)
+        v = torch.randn(n, 2, 128, generator=torch.Generator().manual_seed(n)).to(dtype).to(dev)
+        st.append_chunk(k, v)
+        q = sample_keys(T * 2 * g, seed=n + 1).view(T, 2 * g, 128).to(dev)
+        kr = sample_keys(max(rn, 1) * 2, seed=n + 2).view(-1, 2, 128).to(dtype).to(dev) if rn else None
+        pos = torch.arange(n + rn - T, n + rn, device=dev) if T > 1 else None
+        got = S.compute_hybrid_attention(q, st, kr, kr, 2 * g, query_positions=pos)
+        ref = S.compute_hybrid_attention(q, st, kr, kr, 2 * g, query_positions=pos, impl=1)
+        _close(got, ref, (v,) if kr is None else (v, kr), f"{codec}{size} v{vbits} g{g} T{T} n{n} r{rn}")
+        again = S.compute_hybrid_attention(q, st, kr, kr, 2 * g, query_positions=pos)
+        assert torch.equal(got, again)
+
+
+@pytest.mark.parametrize("codec,size,vbits,g,T,dtype", FORMS[:7:3] + FORMS[4:5])
+@pytest.mark.parametrize("block_size", [0, 16, 64])
+def test_rows_ragged_batches(dev, codec, size, vbits, g, T, dtype, block_size):
+    """Ragged sequences (odd first rows, more than the 64 of one scan step),
+    contiguous or in shuffled pages, then shorter lengths set on the same plan:
+    zero, one token, a part of a page.  The counters are left at zero."""
+    strat = _strategy(dev, codec, size, seed=9)
+    lens = [(37 * i * i) % 389 + 1 for i in range(66)] + [1500]
+    gen = torch.Generator().manual_seed(3)
+    keys = [sample_keys(n * 2, seed=i).view(n, 2, 128).to(dtype).to(dev) for i, n in enumerate(lens)]
+    vals = [torch.randn(n, 2, 128, generator=gen).to(dtype).to(dev) for n in lens]
+    # (N(0, 1) queries reach logits of 366 in the calibrated metric, where either
+    # side is 1.2e-4 off the float64 result: 2^-22 * 366 = 9e-5, times |v|)
+    q = sample_keys(len(lens) * T * 2 * g, seed=99).view(len(lens), T, 2 * g, 128).to(dev)
+    if block_size:
+        need = [-(-n // block_size) for n in lens]
+        perm = torch.randperm(sum(need), generator=gen).to(torch.int32)
+        table = torch.zeros(len(lens), max(need), dtype=torch.int32)
+        for i, (c, part) in enumerate(zip(need, perm.split(need))):
+            table[i, :c] = part
+        kv = PagedQuantizedKV.encode(strat, keys, vals, table.to(dev), sum(need), block_size=block_size, value_bits=vbits)
+    else:
+        kv = QuantizedKVBatch.encode(strat, keys, vals, value_bits=vbits)
+    plans = [kv.plan(q, impl=i) for i in (0, 1)]
+    for cut in (None, torch.tensor([(n * i) % (n + 1) for i, n in enumerate(lens)])):
+        for p in plans:
+            if cut is not None:
+                p.set_lengths(hist_len=cut)
+        got, ref = (p.run(q) for p in plans)
+        _close(got, ref, vals, f"{codec}{size} v{vbits} g{g} T{T} block {block_size} {'cut' if cut is not None else ''}")
+        assert not plans[0].arrivals.any()
+
+
+def test_rows_value_scale_range_and_nan(dev):
+    """Value scales from 2^-24 to 2^15 across tokens (the weights' exponent
+    follows the largest), then a NaN key norm: its row's outputs are NaN."""
+    strat = _strategy(dev, "scalar", 3)
+    n, g = 700, 8
+    v = torch.randn(n, 2, 128, generator=torch.Generator().manual_seed(1))
+    v[100:200] *= 2.0 ** -24
+    v[300:310] *= 2.0 ** 15
+    k = sample_keys(n * 2, seed=2).view(n, 2, 128)
+    kv = QuantizedKVBatch.encode(strat, [k.to(dev)], [v.to(dev)])
+    q = sample_keys(2 * g, seed=3).view(1, 2 * g, 128).to(dev)
+    got, ref = kv.attention(q), kv.attention(q, impl=1)
+    _close(got, ref, (v,), "scales")
+    kv.norms[1, 350] = float("nan")
+    bad = kv.attention(q)
+    assert bool(bad[:, g:].isnan().all()) and torch.equal(bad[:, :g], got[:, :g])
+
+
+def test_rows_small_workspace_runs_generic(dev):
+    """A workspace of the generic kernels' size (sized without arrival
+    counters) is still enough."""
+    import ctypes
+    from smaq_amd import _native
+    strat = _strategy(dev, "vq", 8)
+    n = 400
+    k = sample_keys(n * 2, seed=5).view(n, 2, 128).to(dev)
+    kv = QuantizedKVBatch.encode(strat, [k], [k])
+    q = sample_keys(4, seed=6).view(1, 4, 128).to(dev)
+    plan = kv.plan(q)
+    want = kv.attention(q, impl=1)
+    arrivals, plan.params.arrivals = plan.params.arrivals, None
+    small = _native.lib().smaq_attn_workspace_bytes(ctypes.byref(plan.params))
+    plan.params.arrivals = arrivals
+    assert small < plan.params.workspace_bytes
+    plan.params.workspace_bytes = small
+    assert torch.equal(plan.run(q).view_as(want), want)
