@@ -475,6 +475,14 @@ constexpr int kDecodeMaxPieces = 8;
 
 static int64_t align256(int64_t x) { return (x + 255) & ~(int64_t)255; }
 
+// Bytes of the partials (m, l, o).
+static int64_t partial_bytes(const smaq_attn_params* p, const Plan& pl) {
+  const int64_t S = pl.s_hist + pl.s_recent;
+  const int64_t rows = (int64_t)p->q_len * (p->n_q_heads / p->n_kv_heads);
+  const int64_t n = (int64_t)p->batch * p->n_kv_heads * rows * (S > 0 ? S : 1);
+  return n * (p->head_dim + 2) * (int64_t)sizeof(float);
+}
+
 static Plan make_plan(const smaq_attn_params* p, bool allow_rows) {
   Plan pl;
   const int g = p->n_q_heads / p->n_kv_heads;
@@ -485,7 +493,8 @@ static Plan make_plan(const smaq_attn_params* p, bool allow_rows) {
   // The row kernel merges the recent window's partials, so that phase has to
   // be in the same call.  It wins wherever it is supported: 37x at 16 x 32768
   // tokens, 43x at 64 paged sequences (attention_rows.h), 2.9x for the whole
-  // call at 5 query tokens over 4001, 3x at 16 tokens.
+  // call at 5 query tokens over 4001, and down to 16 tokens (28/4 heads, plan
+  // alone: 33 against 46 us of scalar keys, 23 against 37 of block-VQ).
   const int phase_mask = p->phases ? p->phases : 15;
   pl.rows = allow_rows && !pl.mfma && !pl.prefill && rows_supported(*p) &&
             (!p->has_recent || p->max_recent_len <= 0 || (phase_mask & 3) == 3);
@@ -499,7 +508,7 @@ static Plan make_plan(const smaq_attn_params* p, bool allow_rows) {
   if (pl.mfma) split = mfma_decode_split_len(*p);
   pl.hist_split = split;
   int64_t rl = p->has_recent ? p->max_recent_len : 0;
-  pl.recent_split = (!pl.prefill && recent_decode_supported(*p)) ? recent_decode_split_len() : 4 * kChunk;
+  pl.recent_split = 4 * kChunk;
   pl.hist_lp = pl.recent_lp = 0;
   if (pl.prefill) {
     if (hl > 0) pl.hist_split = prefill_split_len(*p, hl);
@@ -509,6 +518,15 @@ static Plan make_plan(const smaq_attn_params* p, bool allow_rows) {
   }
   pl.s_hist = hl > 0 && !pl.rows ? (int)((hl + pl.hist_split - 1) / pl.hist_split) : 0;
   pl.s_recent = rl > 0 ? (int)((rl + pl.recent_split - 1) / pl.recent_split) : 0;
+  // The decode recent kernel's one-chunk splits, unless their partials alone
+  // pass the built-in scratch's size (with several row tiles: what fitted
+  // there still fits).
+  if (rl > 0 && !pl.prefill && recent_decode_supported(*p)) {
+    Plan fine = pl;
+    fine.recent_split = recent_decode_split_len();
+    fine.s_recent = (int)((rl + fine.recent_split - 1) / fine.recent_split);
+    if (recent_one_tile(*p) || partial_bytes(p, fine) <= SMAQ_NOALLOC_SCRATCH_BYTES / 2) pl = fine;
+  }
   // With ragged lengths and a single split per sequence the workgroups differ
   // in length by up to max / min; dispatched in batch order, the long ones
   // that start late leave the GPU mostly idle at the end (measured: 256
@@ -543,14 +561,6 @@ static Plan make_plan(const smaq_attn_params* p, bool allow_rows) {
 // (16 bytes each).
 static int64_t order_bytes(const smaq_attn_params* p, const Plan& pl) {
   return pl.n_items > 0 ? (int64_t)pl.n_items * 16 : (int64_t)p->batch * (int64_t)sizeof(int);
-}
-
-// Bytes of the partials (m, l, o) and the offset of the longest-first order.
-static int64_t partial_bytes(const smaq_attn_params* p, const Plan& pl) {
-  const int64_t S = pl.s_hist + pl.s_recent;
-  const int64_t rows = (int64_t)p->q_len * (p->n_q_heads / p->n_kv_heads);
-  const int64_t n = (int64_t)p->batch * p->n_kv_heads * rows * (S > 0 ? S : 1);
-  return n * (p->head_dim + 2) * (int64_t)sizeof(float);
 }
 
 }  // namespace smaq

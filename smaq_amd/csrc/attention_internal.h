@@ -88,11 +88,13 @@ int launch_prefill_planes_recent(const smaq_attn_params& p, const PrefillPlanes&
 int launch_prefill_mfma(const smaq_attn_params& p, const PrefillPart& pp, int n_splits, const Partials& part,
                         hipStream_t st);
 
-// Recent window of a decode step (attention_recent.hip): one query token per
-// sequence, head_dim 128, 1/2/4 query heads per KV head; impl 1 keeps the
-// generic kernel.  Writes the same partials as the generic recent kernel
-// (splits s_base .. s_base+n_splits-1).
+// Recent window of a decode step (attention_recent.hip): up to 15 query
+// tokens per sequence, head_dim 128; impl 1 keeps the generic kernel.  Writes
+// the same partials as the generic recent kernel (splits s_base ..
+// s_base+n_splits-1).
 bool recent_decode_supported(const smaq_attn_params& p);
+// one query token at 1, 2 or 4 heads per KV head
+bool recent_one_tile(const smaq_attn_params& p);
 // tokens per split of the decode recent window (one chunk per workgroup)
 int64_t recent_decode_split_len();
 int launch_recent_decode(const smaq_attn_params& p, const Partials& part, int s_base, int n_splits,

@@ -1,7 +1,9 @@
-// Exact recent window of a decode step (one query token per sequence,
-// head_dim 128, 1, 2 or 4 query heads per KV head): the partials of the
-// window's tokens for one (split, KV head, sequence), as the generic recent
-// kernel in attention.hip writes them, from wide coalesced loads.
+// Exact recent window of a decode step (up to 15 query tokens per sequence,
+// head_dim 128): the partials of the window's tokens for one (split, KV head,
+// tile of query rows, sequence), as the generic recent kernel in
+// attention.hip writes them, from wide coalesced loads.  One query token at
+// 1, 2 or 4 heads per KV head is one tile of that many rows; any other number
+// of rows (query tokens x heads per KV head) runs in tiles of 8.
 //
 // Reference: the recent segment of compute_hybrid_attention
 // (smaq/score.py:61-72): scores q . k * scale in fp32 against the exact keys,
@@ -18,7 +20,10 @@
 // 256-byte value row per wave load).  The chunk's key and value loads are all
 // issued before any is used, and the first chunk's together with the
 // window length and the query rows, so a one-chunk split costs one memory
-// round trip.
+// round trip.  Latency bounds it.  The tiles of 8 rows, whole call before (the
+// generic kernel: a row's keys element by element, 90-110 us) and now: 128
+// tokens at 28/4 heads beside 65408 of history 128 -> 47.6 us, 5 query tokens
+// at 32/8 heads over 100 tokens beside 4001 141 -> 42.1 us.
 #include <math.h>
 
 #include "attention_internal.h"
@@ -82,13 +87,26 @@ struct RecentLds {
   __attribute__((aligned(16))) float qs[G][kRD];  // the query rows
   float sc[G][kRChunk];                            // the chunk's scores, then weights
   float m_s[G], l_s[G], a_s[G];
+  long long qpos[G];                               // causal positions of the rows
   float red[4][G][kRD];                            // per-wave outputs, summed at the end
 };
 
-// Split s of the window of (KV head h, sequence b); tid = thread index.
+// Split s of the window of (KV head and row tile ht, sequence b); tid = thread
+// index.
 template <typename TR, int G>
 __device__ __forceinline__ void recent_block(RecentLds<G>& L, const smaq_attn_params& p, const Partials& part,
-                                             int s_base, int64_t split_len, int s, int h, int b, int tid) {
+                                             int s_base, int64_t split_len, int s, int ht, int b, int tid) {
+  const int grp = p.n_q_heads / p.n_kv_heads;
+  const int rows = G == 8 ? p.q_len * grp : G, tiles = (rows + G - 1) / G;
+  const int h = G == 8 ? ht / tiles : ht, r0 = G == 8 ? (ht - h * tiles) * G : 0;
+  const int nr = G == 8 ? min(G, rows - r0) : G;  // live rows of the tile
+  // query token and element offset of the tile's row g (a row past the last
+  // repeats the first, and is dropped)
+  auto token_of = [&](int g) -> int { return G == 8 ? (r0 + (g < nr ? g : 0)) / grp : 0; };
+  auto row_off = [&](int g) -> int64_t {
+    const int row = r0 + (g < nr ? g : 0), t = G == 8 ? row / grp : 0;
+    return (((int64_t)b * p.q_len + t) * p.n_q_heads + (int64_t)h * grp + (row - t * grp)) * kRD;
+  };
   auto& qs = L.qs;
   auto& sc = L.sc;
   auto& m_s = L.m_s;
@@ -118,15 +136,14 @@ __device__ __forceinline__ void recent_block(RecentLds<G>& L, const smaq_attn_pa
   load_chunk(t0);
   const int64_t len = p.recent_len ? min((int64_t)p.recent_len[b], (int64_t)p.max_recent_len) : p.max_recent_len;
   const int64_t t1 = min(len, t0 + split_len);
-  const long long qpos = p.q_positions ? p.q_positions[b] : 0;
 
-  // the G query rows of this KV head, staged in LDS (lane (tq, dq) reads
+  // the G query rows of this tile, staged in LDS (lane (tq, dq) reads
   // dims 32 dq .. of each)
-  for (int i = tid; i < G * kRD; i += 256)
-    qs[i / kRD][i % kRD] = exact_query(p, ((int64_t)b * p.n_q_heads + h * G) * kRD + i);
+  for (int i = tid; i < G * kRD; i += 256) qs[i / kRD][i % kRD] = exact_query(p, row_off(i / kRD) + i % kRD);
   if (tid < G) {
     m_s[tid] = -__builtin_inff();
     l_s[tid] = 0.0f;
+    L.qpos[tid] = p.q_positions ? p.q_positions[(int64_t)b * p.q_len + token_of(tid)] : 0x7fffffffffffffffll;
   }
   float o[G][2];
 #pragma unroll
@@ -158,24 +175,27 @@ __device__ __forceinline__ void recent_block(RecentLds<G>& L, const smaq_attn_pa
       acc[g] += __shfl_xor(acc[g], 32, 64);
     }
     if (dq == 0) {
-      const bool live = kt < nt && !(p.q_positions && p.recent_pos_offset + c0 + kt > qpos);
 #pragma unroll
-      for (int g = 0; g < G; ++g) sc[g][kt] = live ? acc[g] * p.scale : -__builtin_inff();
+      for (int g = 0; g < G; ++g) {
+        const bool live = kt < nt && !(p.q_positions && p.recent_pos_offset + c0 + kt > L.qpos[g]);
+        sc[g][kt] = live ? acc[g] * p.scale : -__builtin_inff();
+      }
     }
     __syncthreads();
-    // online softmax of row g by wave g
-    if (w < G) {
-      const float x = sc[w][lane];
-      const float m_old = m_s[w];
+    // online softmax of row g by wave g % 4
+#pragma unroll
+    for (int g = w; g < G; g += 4) {
+      const float x = sc[g][lane];
+      const float m_old = m_s[g];
       const float m_new = fmaxf(m_old, warp_max(x));
       const float pw = m_new == -__builtin_inff() ? 0.0f : __expf(x - m_new);
       const float alpha = m_old == -__builtin_inff() ? 0.0f : __expf(m_old - m_new);
       const float ls = warp_sum(pw);
-      sc[w][lane] = pw;
+      sc[g][lane] = pw;
       if (lane == 0) {
-        l_s[w] = l_s[w] * alpha + ls;
-        m_s[w] = m_new;
-        a_s[w] = alpha;
+        l_s[g] = l_s[g] * alpha + ls;
+        m_s[g] = m_new;
+        a_s[g] = alpha;
       }
     }
     __syncthreads();
@@ -210,7 +230,8 @@ __device__ __forceinline__ void recent_block(RecentLds<G>& L, const smaq_attn_pa
   for (int i = tid; i < G * kRD; i += 256) {
     const int g = i / kRD, d = i - g * kRD;
     const float sum = (red[0][g][d] + red[1][g][d]) + (red[2][g][d] + red[3][g][d]);
-    const int64_t pi = part.idx(b, h, p.n_kv_heads, G, g, s_base + s);
+    if (g >= nr) continue;
+    const int64_t pi = part.idx(b, h, p.n_kv_heads, rows, r0 + g, s_base + s);
     part.o[pi * kRD + d] = sum;
     if (d == 0) {
       part.m[pi] = m_s[g];
@@ -229,8 +250,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kRecentWave
 // The query rotation (into q_hist) and the recent window in one launch: they
 // are independent (the window reads the raw query), so the shorter one runs
 // beside the longer instead of after it.  Blocks [0, n_rot) rotate 4 rows
-// each (rotate128.h); block n_rot + ((b * Hkv + h) * n_splits + s) takes split
-// s of (KV head h, sequence b).
+// each (rotate128.h); block n_rot + ((b * heads + ht) * n_splits + s) takes split
+// s of (KV head and row tile ht, sequence b).
 template <typename TR, int G>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kRecentWaves<TR>, kRecentWaves<TR>))) void rotate_recent_kernel(
     smaq_attn_params p, Partials part, int s_base, int n_splits, int64_t split_len, int n_rot) {
@@ -246,17 +267,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kRecentWave
   }
   const int r = bx - n_rot;
   const int s = r % n_splits, hb = r / n_splits;
-  recent_block<TR, G>(lds.r, p, part, s_base, split_len, s, hb % p.n_kv_heads, hb / p.n_kv_heads, tid);
+  const int heads = p.n_kv_heads * (G == 8 ? (p.q_len * (p.n_q_heads / p.n_kv_heads) + G - 1) / G : 1);
+  recent_block<TR, G>(lds.r, p, part, s_base, split_len, s, hb % heads, hb / heads, tid);
+}
+
+// rows of a tile: a decode step's heads per KV head, else 8
+int tile_rows(const smaq_attn_params& p) {
+  const int g = p.n_q_heads / p.n_kv_heads;
+  return p.q_len == 1 && (g == 1 || g == 2 || g == 4) ? g : 8;
+}
+// (KV head, row tile) pairs
+int64_t tile_heads(const smaq_attn_params& p) {
+  const int g = p.n_q_heads / p.n_kv_heads, t = tile_rows(p);
+  return (int64_t)p.n_kv_heads * (((int64_t)p.q_len * g + t - 1) / t);
 }
 
 template <typename TR>
 void launch_g(const smaq_attn_params& p, const Partials& part, int s_base, int n_splits, int64_t split_len,
               hipStream_t st) {
-  const dim3 grid((unsigned)n_splits, (unsigned)p.n_kv_heads, (unsigned)p.batch);
-  switch (p.n_q_heads / p.n_kv_heads) {
+  const dim3 grid((unsigned)n_splits, (unsigned)tile_heads(p), (unsigned)p.batch);
+  switch (tile_rows(p)) {
     case 1: hipLaunchKernelGGL((recent_decode_kernel<TR, 1>), grid, dim3(256), 0, st, p, part, s_base, split_len); break;
     case 2: hipLaunchKernelGGL((recent_decode_kernel<TR, 2>), grid, dim3(256), 0, st, p, part, s_base, split_len); break;
-    default: hipLaunchKernelGGL((recent_decode_kernel<TR, 4>), grid, dim3(256), 0, st, p, part, s_base, split_len); break;
+    case 4: hipLaunchKernelGGL((recent_decode_kernel<TR, 4>), grid, dim3(256), 0, st, p, part, s_base, split_len); break;
+    default: hipLaunchKernelGGL((recent_decode_kernel<TR, 8>), grid, dim3(256), 0, st, p, part, s_base, split_len); break;
   }
 }
 
@@ -264,9 +298,11 @@ void launch_g(const smaq_attn_params& p, const Partials& part, int s_base, int n
 
 int64_t recent_decode_split_len() { return kRChunk; }
 
+bool recent_one_tile(const smaq_attn_params& p) { return p.q_len == 1 && tile_rows(p) < 8; }
+
 bool recent_decode_supported(const smaq_attn_params& p) {
-  const int g = p.n_q_heads / p.n_kv_heads;
-  return p.impl != 1 && p.has_recent && p.q_len == 1 && p.head_dim == kRD && (g == 1 || g == 2 || g == 4) &&
+  // (from 16 query tokens on the prefill kernel takes the window)
+  return p.impl != 1 && p.has_recent && p.q_len < 16 && p.head_dim == kRD && tile_heads(p) < 65536 &&
          (p.recent_dtype == SMAQ_F32 || p.recent_dtype == SMAQ_F16 || p.recent_dtype == SMAQ_BF16) &&
          // 16-byte key loads and 4- or 8-byte value loads at element offsets
          // that are multiples of 8 and 2
@@ -278,11 +314,12 @@ void launch_rg(const smaq_attn_params& p, const Partials& part, int s_base, int 
                hipStream_t st) {
   const int64_t rows = (int64_t)p.batch * p.q_len * p.n_q_heads;
   const int n_rot = (int)((rows + 3) / 4);
-  const dim3 grid((unsigned)(n_rot + (int64_t)n_splits * p.n_kv_heads * p.batch));
-  switch (p.n_q_heads / p.n_kv_heads) {
+  const dim3 grid((unsigned)(n_rot + (int64_t)n_splits * tile_heads(p) * p.batch));
+  switch (tile_rows(p)) {
     case 1: hipLaunchKernelGGL((rotate_recent_kernel<TR, 1>), grid, dim3(256), 0, st, p, part, s_base, n_splits, split_len, n_rot); break;
     case 2: hipLaunchKernelGGL((rotate_recent_kernel<TR, 2>), grid, dim3(256), 0, st, p, part, s_base, n_splits, split_len, n_rot); break;
-    default: hipLaunchKernelGGL((rotate_recent_kernel<TR, 4>), grid, dim3(256), 0, st, p, part, s_base, n_splits, split_len, n_rot); break;
+    case 4: hipLaunchKernelGGL((rotate_recent_kernel<TR, 4>), grid, dim3(256), 0, st, p, part, s_base, n_splits, split_len, n_rot); break;
+    default: hipLaunchKernelGGL((rotate_recent_kernel<TR, 8>), grid, dim3(256), 0, st, p, part, s_base, n_splits, split_len, n_rot); break;
   }
 }
 
@@ -290,7 +327,7 @@ bool rotate_recent_supported(const smaq_attn_params& p) {
   const int64_t rows = (int64_t)p.batch * p.q_len * p.n_q_heads;
   return recent_decode_supported(p) && p.rot_mt && p.q_raw && p.q_hist && ((uintptr_t)p.rot_mt & 15) == 0 &&
          (p.q_raw_dtype == SMAQ_F32 || p.q_raw_dtype == SMAQ_F16 || p.q_raw_dtype == SMAQ_BF16) &&
-         (rows + 3) / 4 + (int64_t)p.n_kv_heads * p.batch * 64 < (1ll << 31);
+         (rows + 3) / 4 + tile_heads(p) * p.batch * 64 < (1ll << 31);
 }
 
 int launch_rotate_recent(const smaq_attn_params& p, const Partials& part, int s_base, int n_splits,
