@@ -142,6 +142,20 @@ int smaq_encode_blockvq(const void* k, int kdtype, long long n_outer, long long 
                         void* idx_out, unsigned long long* tie_count, void* stream);
 
 /*
+ * smaq_encode_blockvq with a workspace (16-byte aligned; NULL: none) of
+ * smaq_encode_blockvq_workspace_bytes (0: none is used): the same indices and
+ * tie counts.  With 2-dim blocks each call first writes, for every cell of a
+ * grid over a block's plane, the centroids that can be nearest to a point of
+ * it, and the argmin then runs over those.
+ */
+long long smaq_encode_blockvq_workspace_bytes(int n_blocks, int block_dim, int n_centroids);
+int smaq_encode_blockvq_ws(const void* k, int kdtype, long long n_outer, long long n_inner,
+                           long long s_outer, long long s_inner, long long out_outer, int n_blocks, int block_dim,
+                           int n_centroids, const float* E_blocks, const float* centroids,
+                           void* idx_out, unsigned long long* tie_count, void* workspace,
+                           long long workspace_bytes, void* stream);
+
+/*
  * Block-VQ dequantiser.  Replaces SMAQBlockVQ.dequantize (smaq/block_vq.py:246-267):
  * k_hat[r, b*bd + i] = decoded[b][idx[r, b]][i] (fp32).
  */

@@ -76,6 +76,9 @@ _SIGS = {
                                    c_int, c_void_p, c_int, c_float, c_void_p, c_int, c_void_p]),
     "smaq_encode_blockvq": (c_int, [c_void_p, c_int, c_ll, c_ll, c_ll, c_ll, c_ll, c_int, c_int, c_int,
                                     c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "smaq_encode_blockvq_workspace_bytes": (c_ll, [c_int, c_int, c_int]),
+    "smaq_encode_blockvq_ws": (c_int, [c_void_p, c_int, c_ll, c_ll, c_ll, c_ll, c_ll, c_int, c_int, c_int,
+                                       c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_ll, c_void_p]),
     "smaq_dequant_blockvq": (c_int, [c_void_p, c_ll, c_int, c_int, c_int, c_void_p, c_void_p,
                                      c_void_p]),
     "smaq_blockvq_shape": (c_int, [c_void_p, c_int, c_ll, c_int, c_int, c_void_p, c_void_p, c_void_p]),
@@ -449,8 +452,11 @@ def encode_blockvq(k: torch.Tensor, E_blocks: torch.Tensor, centroids: torch.Ten
         idx = out
     eb = E_blocks.to(torch.float32).contiguous()
     cents = centroids.to(torch.float32).contiguous()
-    _check(lib().smaq_encode_blockvq(_ptr(k), dtype_code(k.dtype), no, ni, so, si, oo, nb, bd, nc, _ptr(eb),
-                                     _ptr(cents), _ptr(idx), ties.ptr() if ties else None, _stream(dev)),
+    ws_bytes = lib().smaq_encode_blockvq_workspace_bytes(nb, bd, nc)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
+    _check(lib().smaq_encode_blockvq_ws(_ptr(k), dtype_code(k.dtype), no, ni, so, si, oo, nb, bd, nc, _ptr(eb),
+                                        _ptr(cents), _ptr(idx), ties.ptr() if ties else None, _ptr(ws), ws_bytes,
+                                        _stream(dev)),
            "smaq_encode_blockvq")
     return idx
 

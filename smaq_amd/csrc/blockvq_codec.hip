@@ -123,6 +123,21 @@ extern "C" int smaq_encode_blockvq(const void* k, int kdtype, long long n_outer,
                                    int block_dim, int n_centroids, const float* E_blocks,
                                    const float* centroids, void* idx_out,
                                    unsigned long long* tie_count, void* stream) {
+  return smaq_encode_blockvq_ws(k, kdtype, n_outer, n_inner, s_outer, s_inner, out_outer, n_blocks, block_dim,
+                                n_centroids, E_blocks, centroids, idx_out, tie_count, nullptr, 0, stream);
+}
+
+extern "C" long long smaq_encode_blockvq_workspace_bytes(int n_blocks, int block_dim, int n_centroids) {
+  return block_dim == 2 && n_blocks > 0 && n_blocks % 4 == 0 && n_centroids > 64 && n_centroids <= 256
+             ? encode_2d_bytes(n_blocks)
+             : 0;
+}
+
+extern "C" int smaq_encode_blockvq_ws(const void* k, int kdtype, long long n_outer, long long n_inner,
+                                      long long s_outer, long long s_inner, long long out_outer, int n_blocks,
+                                      int block_dim, int n_centroids, const float* E_blocks,
+                                      const float* centroids, void* idx_out, unsigned long long* tie_count,
+                                      void* workspace, long long workspace_bytes, void* stream) {
   SMAQ_REQUIRE(k && E_blocks && centroids && idx_out, "smaq_encode_blockvq: null pointer");
   SMAQ_REQUIRE(block_dim >= 1 && block_dim <= kVqMaxBlockDim,
                "smaq_encode_blockvq: block_dim must be in [1, %d], got %d", kVqMaxBlockDim,
@@ -142,6 +157,14 @@ extern "C" int smaq_encode_blockvq(const void* k, int kdtype, long long n_outer,
   if (encode_blockvq_mfma_supported(n_blocks, block_dim, n_centroids, k, kdtype, s_outer, s_inner))
     return launch_encode_blockvq_mfma(kdtype, k, map, rows, n_blocks, E_blocks, centroids,
                                       (uint8_t*)idx_out, tie_count, st);
+  // (261,632 fp16 rows of 64 blocks: 142 us, 10,920 us with the scan below; with
+  // few centroids the scan is short, and a list could hold all of them)
+  if (workspace && workspace_bytes >= encode_2d_bytes(n_blocks) &&
+      (kdtype == SMAQ_F32 || kdtype == SMAQ_F16 || kdtype == SMAQ_BF16) &&
+      encode_2d_supported(n_blocks, block_dim, n_centroids, rows, k, kdtype, s_outer, s_inner, n_inner, centroids,
+                          idx_out, workspace))
+    return launch_encode_2d(kdtype, k, map, rows, n_blocks, n_centroids, E_blocks, centroids, (uint8_t*)idx_out,
+                            tie_count, workspace, st);
   const size_t lds = (size_t)n_blocks * n_centroids * sizeof(float);
   const unsigned grid = (unsigned)((rows + kVqThreads - 1) / kVqThreads);
   switch (kdtype) {

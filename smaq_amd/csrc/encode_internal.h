@@ -35,6 +35,14 @@ int launch_encode_scalar_mfma(int kdtype, const void* k, RowMap map, int64_t row
 bool encode_blockvq_mfma_supported(int nb, int bd, int nc, const void* k, int kdtype,
                                    long long s_outer, long long s_inner);
 size_t encode_blockvq_mfma_lds(int nb);
+
+// Block-VQ encoder for 2-dim blocks (blockvq_encode_2d.hip): 65 to 256
+// centroids, a multiple of 4 blocks, encode_2d_bytes of workspace.
+bool encode_2d_supported(int nb, int bd, int nc, int64_t rows, const void* k, int kdtype, long long s_outer,
+                         long long s_inner, long long n_inner, const void* C, const void* idx, const void* ws);
+int64_t encode_2d_bytes(int nb);
+int launch_encode_2d(int kdtype, const void* k, RowMap map, int64_t rows, int nb, int nc, const float* E_blocks,
+                     const float* C, uint8_t* idx, unsigned long long* ties, void* ws, hipStream_t st);
 int launch_encode_blockvq_mfma(int kdtype, const void* k, RowMap map, int64_t rows, int nb,
                                const float* E_blocks, const float* C, uint8_t* idx,
                                unsigned long long* ties, hipStream_t st);

@@ -483,3 +483,65 @@ def test_scalar_encode_cancellation_matches_the_chain(dev, dtype):
     assert int(near.sum()) > 100          # the construction exercises the recount
     assert torch.equal(got.indices.cpu(), ref.indices)
     assert torch.equal(got.norms.cpu(), ref.norms)
+
+
+# ------------------------------------- block VQ, 2-dim blocks (cell lists) ---
+
+def _encode_2d(dev, k, E, C, listed: bool):
+    """(indices, tie count) through the cell lists, or through the full scan
+    (no workspace)."""
+    from smaq_amd import _native as N
+    n, nb, nc = k.shape[0], C.shape[0], C.shape[1]
+    idx = torch.full((n, nb), 255, dtype=torch.uint8, device=dev)
+    ties = N.TieCounter(dev)
+    size = N.lib().smaq_encode_blockvq_workspace_bytes(nb, 2, nc) if listed else 0
+    ws = torch.empty(size, dtype=torch.uint8, device=dev).fill_(0xA5) if listed else None
+    assert (size > 0) == listed
+    rc = N.lib().smaq_encode_blockvq_ws(N._ptr(k), N.dtype_code(k.dtype), 1, n, 0, k.stride(0), 0, nb, 2, nc, N._ptr(E),
+                                        N._ptr(C), N._ptr(idx), ties.ptr(), N._ptr(ws), size, N._stream(dev))
+    assert rc == 0
+    return idx, ties.value()
+
+
+@pytest.mark.parametrize("nc,dtype,rows", [(256, torch.float16, 5000), (256, torch.bfloat16, 1), (100, torch.float32, 1025),
+                                           (65, torch.bfloat16, 63), (130, torch.float16, 64)])
+@pytest.mark.parametrize("shape", ["gauss", "narrow", "ties", "far", "flat", "nonfinite"])
+def test_blockvq_2d_lists_match_the_scan(dev, nc, dtype, rows, shape):
+    """Indices and tie counts of the cell lists equal the full scan's, bit for
+    bit: Gaussian blocks; one axis 50 times the other; duplicated centroids
+    and keys on centroids and half way between two; keys far outside; all
+    centroids on a line or equal; NaN and infinite keys and centroids."""
+    g = torch.Generator().manual_seed(nc + rows)
+    nb = 16
+    C = torch.randn(nb, nc, 2, generator=g)
+    k = torch.randn(rows, nb, 2, generator=g) * 1.2
+    E = torch.eye(2).repeat(nb, 1, 1) + 0.2 * torch.randn(nb, 2, 2, generator=g)
+    if shape == "narrow":
+        C[..., 0] *= 50
+        k[..., 0] *= 50
+        C += 3.0
+        k += 3.0
+    elif shape == "ties":
+        E = torch.eye(2).repeat(nb, 1, 1)
+        C = (C * 4).round() / 4
+        k = (k * 8).round() / 8
+    elif shape == "far":
+        k[::3] *= 1000
+        k[1::7] *= 1e-6
+        C[:, ::2] *= 30
+    elif shape == "flat":
+        C[:8, :, 1] = 0.5
+        C[8:] = C[8:, :1]
+    elif shape == "nonfinite":
+        k[::5, 3, 0] = float("nan")
+        k[::4, 5, 1] = float("inf")
+        C[7, nc // 2, 0] = float("nan")
+        C[9, 0, 1] = float("inf")
+        C[11] *= 1e20
+    k = k.reshape(rows, 2 * nb).to(dtype).to(dev)
+    C, E = C.contiguous().to(dev), E.contiguous().to(dev)
+    want, ties = _encode_2d(dev, k, E, C, False)
+    got, got_ties = _encode_2d(dev, k, E, C, True)
+    bad = (got != want).sum().item()
+    assert bad == 0, f"{bad} of {want.numel()} indices differ"
+    assert got_ties == ties
