@@ -207,8 +207,16 @@ __device__ int exact_argmin(const float* x, float xsq, const float* __restrict__
 
 template <typename T>
 __global__ __launch_bounds__(kVmThreads) void encode_blockvq_mfma_kernel(
-    const T* __restrict__ k, RowMap map, int64_t rows, int nb, const float* __restrict__ E_blocks,
+    const T* __restrict__ k, RowMap map, int64_t rows, int nb, int nb_row, const float* __restrict__ E_blocks,
     const float* __restrict__ C, uint8_t* __restrict__ idx_out, unsigned long long* tie_count) {
+  // this workgroup's blocks: nb of the row's nb_row
+  {
+    const int b0 = blockIdx.y * nb;
+    k += b0 * kVmBd;
+    E_blocks += b0 * kVmBd * kVmBd;
+    C += (int64_t)b0 * kVmNc * kVmBd;
+    idx_out += b0;
+  }
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const VmLds L{nb};
   float* const es_all = (float*)(lds + L.es());
@@ -324,7 +332,7 @@ __global__ __launch_bounds__(kVmThreads) void encode_blockvq_mfma_kernel(
   for (; set < n_sets; set += stride) {
     const int64_t row = set * 64 + lane;  // the token this lane finishes
     const bool valid = row < rows;
-    uint8_t* const out = idx_out + map.out_row(valid ? row : 0) * nb;
+    uint8_t* const out = idx_out + map.out_row(valid ? row : 0) * nb_row;
     // the token's indices, byte b in word b / 4, stored together after the
     // last block (one store per block and token leaves 16 partial writes of
     // a row to reach HBM separately once the set's rows fall out of L2)
@@ -484,6 +492,8 @@ __global__ __launch_bounds__(kVmThreads) void encode_blockvq_mfma_kernel(
     if (valid) {
       if (nb == kVmMaxBlocks && ((uintptr_t)out & 15) == 0) {
         *(u32x4*)out = u32x4{ob[0], ob[1], ob[2], ob[3]};
+      } else if (nb == 4 && ((uintptr_t)out & 3) == 0) {
+        *(uint32_t*)out = ob[0];
       } else {
         for (int b = 0; b < nb; ++b) out[b] = (uint8_t)(ob[b >> 2] >> (8 * (b & 3)));
       }
@@ -512,10 +522,17 @@ int launch_encode_blockvq_mfma(int kdtype, const void* k, RowMap map, int64_t ro
   int dev = 0, cus = 256;
   if (hipGetDevice(&dev) == hipSuccess)
     hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  const int64_t n_tiles = (rows + 15) / 16;
-  const int64_t want = (n_tiles + kVmWaves - 1) / kVmWaves;
-  const unsigned grid = (unsigned)(want < cus ? want : cus);
-  const size_t lds = encode_blockvq_mfma_lds(nb);
+  const int64_t n_sets = (rows + 63) / 64;
+  const int64_t want = (n_sets + kVmWaves - 1) / kVmWaves;
+  // Few rows: a row's blocks are divided among workgroups, which splits the
+  // codebook's preparation (156 KB of LDS for 16 blocks, most of a small call)
+  // and fills the device.  16 bf16 blocks, together and divided: 128 rows 49.5
+  // and 13.8 us, 1,024 rows 125 and 16.5, 16,376 129 and 18.5, 65,536 131 and
+  // 43, 131,072 136 and 77; from 131,073 rows on they stay together.
+  int per = nb;
+  while (per > 1 && per % 2 == 0 && want * (nb / per) * 2 <= cus) per /= 2;
+  const dim3 grid((unsigned)(want < cus ? want : cus), (unsigned)(nb / per));
+  const size_t lds = encode_blockvq_mfma_lds(per);
   // the split codebook takes more than the default 64 KB of dynamic LDS
   switch (kdtype) {
     case SMAQ_F32:
@@ -533,16 +550,16 @@ int launch_encode_blockvq_mfma(int kdtype, const void* k, RowMap map, int64_t ro
   }
   switch (kdtype) {
     case SMAQ_F32:
-      hipLaunchKernelGGL(encode_blockvq_mfma_kernel<float>, dim3(grid), dim3(kVmThreads), lds, st,
-                         (const float*)k, map, rows, nb, E_blocks, C, idx, ties);
+      hipLaunchKernelGGL(encode_blockvq_mfma_kernel<float>, grid, dim3(kVmThreads), lds, st,
+                         (const float*)k, map, rows, per, nb, E_blocks, C, idx, ties);
       break;
     case SMAQ_F16:
-      hipLaunchKernelGGL(encode_blockvq_mfma_kernel<_Float16>, dim3(grid), dim3(kVmThreads), lds, st,
-                         (const _Float16*)k, map, rows, nb, E_blocks, C, idx, ties);
+      hipLaunchKernelGGL(encode_blockvq_mfma_kernel<_Float16>, grid, dim3(kVmThreads), lds, st,
+                         (const _Float16*)k, map, rows, per, nb, E_blocks, C, idx, ties);
       break;
     default:
-      hipLaunchKernelGGL(encode_blockvq_mfma_kernel<bf16>, dim3(grid), dim3(kVmThreads), lds, st,
-                         (const bf16*)k, map, rows, nb, E_blocks, C, idx, ties);
+      hipLaunchKernelGGL(encode_blockvq_mfma_kernel<bf16>, grid, dim3(kVmThreads), lds, st,
+                         (const bf16*)k, map, rows, per, nb, E_blocks, C, idx, ties);
       break;
   }
   return launch_status("smaq_encode_blockvq(mfma)");

@@ -545,3 +545,23 @@ def test_blockvq_2d_lists_match_the_scan(dev, nc, dtype, rows, shape):
     bad = (got != want).sum().item()
     assert bad == 0, f"{bad} of {want.numel()} indices differ"
     assert got_ties == ties
+
+
+@pytest.mark.parametrize("nb", [16, 12, 5])
+def test_blockvq_divided_rows_match_the_whole(dev, nb):
+    """Few rows divide a row's blocks among workgroups: slices of a large call
+    (whole rows per workgroup) encode to its indices, ties counted alike."""
+    g = torch.Generator(device=dev).manual_seed(nb)
+    rows, D = 270000, 8 * nb
+    k = torch.randn(rows, D, generator=g, device=dev).bfloat16()
+    C = torch.randn(nb, 256, 8, generator=g, device=dev)
+    E = torch.eye(8, device=dev).repeat(nb, 1, 1).contiguous()
+    t_all = _native.TieCounter(dev)
+    whole = _native.encode_blockvq(k, E, C, ties=t_all)
+    t_cut, at = _native.TieCounter(dev), 0
+    for n in (1, 63, 1500, 9000, 40000, 100000):
+        part = _native.encode_blockvq(k[at:at + n], E, C, ties=t_cut)
+        assert torch.equal(part, whole[at:at + n]), n
+        at += n
+    _native.encode_blockvq(k[at:], E, C, ties=t_cut)
+    assert t_cut.value() == t_all.value()
