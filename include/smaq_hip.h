@@ -289,9 +289,13 @@ typedef struct smaq_attn_params {
   /* kernel choice: 0 = automatic (matrix-core decode kernel when the shape
      allows, generic kernels otherwise), 1 = generic kernels only, 2 = the
      matrix-core decode kernel, 3 = the matrix-core prefill kernel
-     (SMAQ_EUNSUPPORTED if the shape does not fit).  Automatic choice: the
-     decode kernel for single-token queries, the prefill kernel for
-     q_len >= 16 at head_dim 128, the generic kernels otherwise. */
+     (SMAQ_EUNSUPPORTED if the shape does not fit).  Automatic choice at
+     head_dim 128: the decode kernel for single-token queries it serves; with
+     arrival counters (below), block-VQ or 3/4-bit scalar keys and 2- or
+     4-bit values in groups of 32, the matrix-core row kernel for other
+     decode shapes and for fewer than 64 query tokens (from 16 on where it is
+     the faster one); the prefill kernel for q_len >= 16; the generic kernels
+     otherwise. */
   int impl;
   /* Optional split merge inside the matrix-core decode kernel (NULL: a
      combine launch merges the splits).  int32 [batch * Hkv] arrival

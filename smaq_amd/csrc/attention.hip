@@ -496,8 +496,9 @@ static Plan make_plan(const smaq_attn_params* p, bool allow_rows) {
   // call at 5 query tokens over 4001, and down to 16 tokens (28/4 heads, plan
   // alone: 33 against 46 us of scalar keys, 23 against 37 of block-VQ).
   const int phase_mask = p->phases ? p->phases : 15;
-  pl.rows = allow_rows && !pl.mfma && !pl.prefill && rows_supported(*p) &&
+  pl.rows = allow_rows && !pl.mfma && rows_supported(*p) && (!pl.prefill || rows_preferred(*p)) &&
             (!p->has_recent || p->max_recent_len <= 0 || (phase_mask & 3) == 3);
+  if (pl.rows) pl.prefill = false;
   const int64_t units = (int64_t)p->batch * p->n_kv_heads * pl.row_tiles;
   // aim for >= 2048 workgroups over the history
   int64_t want = units >= 2048 ? 1 : (2048 + units - 1) / units;

@@ -88,7 +88,7 @@ int launch_prefill_planes_recent(const smaq_attn_params& p, const PrefillPlanes&
 int launch_prefill_mfma(const smaq_attn_params& p, const PrefillPart& pp, int n_splits, const Partials& part,
                         hipStream_t st);
 
-// Recent window of a decode step (attention_recent.hip): up to 15 query
+// Recent window of a decode step (attention_recent.hip): up to 63 query
 // tokens per sequence, head_dim 128; impl 1 keeps the generic kernel.  Writes
 // the same partials as the generic recent kernel (splits s_base ..
 // s_base+n_splits-1).
@@ -145,12 +145,14 @@ int launch_rotate_schedule(const smaq_attn_params& p, int first_round, int max_p
 int launch_mfma_decode(const smaq_attn_params& p, const HistAddr& a, const Partials& part,
                        int n_splits, bool direct, bool merge, const int* order, int items, hipStream_t st);
 
-// Matrix-core history kernel for up to 15 query tokens (attention_rows.h):
+// Matrix-core history kernel for up to 63 query tokens (attention_rows.h):
 // block-VQ keys, query rows beyond 4 per KV head, 4-bit values.  Needs
 // arrival counters; writes the output itself.  `slots` are rows_bytes of
 // workspace; the `n_recent` partials per row of `recent` (written by the
 // recent launch of the same call) are merged in.
 bool rows_supported(const smaq_attn_params& p);
+// whether it is the faster kernel where the prefill kernel serves the call too
+bool rows_preferred(const smaq_attn_params& p);
 int64_t rows_bytes(const smaq_attn_params& p);
 int launch_rows(const smaq_attn_params& p, const HistAddr& a, void* slots, const Partials& recent, int n_recent,
                 hipStream_t st);

@@ -1,4 +1,4 @@
-// Exact recent window of a decode step (up to 15 query tokens per sequence,
+// Exact recent window of a decode step (up to 63 query tokens per sequence,
 // head_dim 128): the partials of the window's tokens for one (split, KV head,
 // tile of query rows, sequence), as the generic recent kernel in
 // attention.hip writes them, from wide coalesced loads.  One query token at
@@ -301,8 +301,7 @@ int64_t recent_decode_split_len() { return kRChunk; }
 bool recent_one_tile(const smaq_attn_params& p) { return p.q_len == 1 && tile_rows(p) < 8; }
 
 bool recent_decode_supported(const smaq_attn_params& p) {
-  // (from 16 query tokens on the prefill kernel takes the window)
-  return p.impl != 1 && p.has_recent && p.q_len < 16 && p.head_dim == kRD && tile_heads(p) < 65536 &&
+  return p.impl != 1 && p.has_recent && p.q_len < 64 && p.head_dim == kRD && tile_heads(p) < 65536 &&
          (p.recent_dtype == SMAQ_F32 || p.recent_dtype == SMAQ_F16 || p.recent_dtype == SMAQ_BF16) &&
          // 16-byte key loads and 4- or 8-byte value loads at element offsets
          // that are multiples of 8 and 2

@@ -11,7 +11,8 @@
 // count and the raggedness, and a workgroup stages its key table once.  A
 // unit's tokens are thus cut where a share ends; each piece leaves a partial
 // in slot (workgroup + unit), which is unique because either index moves on
-// at every cut, and the last piece to arrive merges the unit in piece order.
+// at every cut, and the last piece to arrive merges the unit in piece order
+// (rows_combine_kernel does, where a KV head has several tiles).
 //
 // Per 32-token tile of a wave (two 16-token halves):
 //   QK   v_mfma_f32_16x16x32_f16, S^T = K q^T: M = 16 tokens, N = 16 columns
@@ -80,6 +81,43 @@ struct RowsRule {
 
 typedef _Float16 rf16x2 __attribute__((ext_vector_type(2)));
 
+// The steps of every unit and how they are dealt to workgroups.
+struct RowsShares {
+  uint32_t total, groups;  // steps; workgroups that have a share
+  uint32_t each, more;     // the first `more` shares hold each + 1 steps, the others `each`
+  __device__ __forceinline__ uint32_t start(uint32_t w) const { return w * each + min(w, more); }
+  // the workgroup whose share holds step y
+  __device__ __forceinline__ uint32_t owner(uint32_t y) const {
+    const uint32_t low = more * (each + 1);
+    return y < low ? y / (each + 1) : more + (y - low) / each;
+  }
+};
+
+__device__ __forceinline__ uint32_t rows_steps(int64_t len, int step) {
+  return len > 0 ? (uint32_t)((len + step - 1) / step) : 1u;
+}
+
+// `before`: the steps of one unit of every sequence below b_end, summed (by
+// the wave; every lane gets it).
+__device__ __forceinline__ uint32_t rows_sum_steps(const smaq_attn_params& p, int step, int b_end, int lane) {
+  if (!p.hist_len) return rows_steps(p.max_hist_len, step) * (uint32_t)b_end;
+  uint32_t sum = 0;
+  for (int b = lane; b < b_end; b += 64)
+    sum += rows_steps(min((int64_t)p.hist_len[b], (int64_t)p.max_hist_len), step);
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) sum += (uint32_t)__shfl_xor((int)sum, o, 64);
+  return (uint32_t)__builtin_amdgcn_readfirstlane(sum);
+}
+
+__device__ __forceinline__ RowsShares rows_shares(const smaq_attn_params& p, const RowsRule& rule, int step, int lane) {
+  RowsShares s;
+  s.total = rows_sum_steps(p, step, p.batch, lane) * (uint32_t)(p.n_kv_heads * rule.tiles);
+  s.groups = min((uint32_t)rule.groups, (s.total + rule.least - 1) / rule.least);
+  s.each = (uint32_t)__builtin_amdgcn_readfirstlane(s.total / s.groups);
+  s.more = s.total - s.each * s.groups;
+  return s;
+}
+
 // x0, x1 -> packed f16 hi pair and packed f16 pair of what it leaves; `one`
 // is an opaque 1.0 (keeps x - hi a mixed-precision FMA)
 __device__ __forceinline__ void rows_split2(float x0, float x1, float one, uint32_t& hi, uint32_t& lo) {
@@ -129,6 +167,121 @@ __device__ __forceinline__ void packed_set(uint32_t* w, int i, T v) {
 constexpr int kRowsPerSimd = 2;
 
 
+// Merge of one unit (query rows of tile ti of KV head h, sequence b): its np
+// partials from `first` on and the recent window's, in that order, by kParts x
+// 256 threads (256: 8 rows x 32 dim quads; with 512 the two halves take
+// alternate pieces).  A merge is a chain of memory round trips, so each has
+// many loads in flight.  `ex`: 11 KB of LDS (kParts 2).
+template <int kParts>
+__device__ __forceinline__ void rows_merge(const smaq_attn_params& p, const RowsRule& rule, const Partials& recent,
+                                           const float* first, int np, int b, int h, int ti, int tid, float* ex) {
+  constexpr int kDeep = 8;
+  constexpr float kLog2e = 1.4426950408889634f;
+  const int g = p.n_q_heads / p.n_kv_heads;
+  const int part = tid >> 8, r = (tid & 255) >> 5, d = 4 * (tid & 31);
+  const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(first), (short)0, -1, 0x00020000);
+  const int row = ti * kRowsQ + r, n_all = np + rule.n_recent;
+  const int64_t rbase =
+      rule.n_recent > 0 ? recent.idx(b, h, p.n_kv_heads, rule.rows, min(row, rule.rows - 1), 0) : 0;
+  float M = -__builtin_inff(), L = 0.0f;
+  f32x4 oh = {0.0f, 0.0f, 0.0f, 0.0f}, orc = oh;
+  bool poisoned = false;  // a partial's sum is NaN
+  for (int c0 = part; c0 < n_all; c0 += kParts * kDeep) {
+    float mv[kDeep], lv[kDeep];
+    f32x4 ov[kDeep];
+#pragma unroll
+    for (int k = 0; k < kDeep; ++k) {
+      const int c = c0 + k * kParts;
+      mv[k] = -__builtin_inff();
+      lv[k] = 0.0f;
+      ov[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      if (c < np) {  // (agent-coherent: written through by the other workgroups)
+        const int off = c * kRowsSlot * 4;
+        mv[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, r * 4, off, kAgentPolicy));
+        lv[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, (kRowsQ + r) * 4, off, kAgentPolicy));
+        ov[k] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                    rs, (2 * kRowsQ + r * 128 + d) * 4, off, kAgentPolicy));
+      } else if (c < n_all) {  // the recent window's partials (natural-log maxima)
+        const int64_t ri = rbase + (c - np);
+        mv[k] = recent.m[ri] * kLog2e;
+        lv[k] = recent.l[ri];
+        ov[k] = *(const f32x4*)&recent.o[ri * 128 + d];
+      }
+    }
+    float Mc = M;
+#pragma unroll
+    for (int k = 0; k < kDeep; ++k) {
+      poisoned |= lv[k] != lv[k];
+      Mc = lv[k] > 0.0f ? fmaxf(Mc, mv[k]) : Mc;
+    }
+    const float c = M == -__builtin_inff() ? 0.0f : fast_exp2(M - Mc);
+    L *= c;
+    oh *= c;
+    orc *= c;
+    M = Mc;
+#pragma unroll
+    for (int k = 0; k < kDeep; ++k) {
+      const bool live = lv[k] > 0.0f;
+      const float wk = live ? fast_exp2(mv[k] - M) : 0.0f;
+      L = live ? fmaf(lv[k], wk, L) : L;
+      const bool hist = c0 + k * kParts < np;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float v = live ? ov[k][i] : 0.0f;
+        oh[i] = fmaf(v, hist ? wk : 0.0f, oh[i]);
+        orc[i] = fmaf(v, hist ? 0.0f : wk, orc[i]);
+      }
+    }
+  }
+  if constexpr (kParts == 2) {
+    __syncthreads();
+    float* const e = ex + (tid & 255);
+    if (part == 1) {
+      e[0] = L;
+      ((uint32_t*)e)[10 * 256] = poisoned ? 1u : 0u;
+      e[256] = M;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        e[(2 + i) * 256] = oh[i];
+        e[(6 + i) * 256] = orc[i];
+      }
+    }
+    __syncthreads();
+    if (part == 0) {
+      const float L2 = e[0], M2 = e[256];
+      poisoned |= ((const uint32_t*)e)[10 * 256] != 0u;
+      const float Mc = fmaxf(M, M2);
+      const float f1 = L > 0.0f ? fast_exp2(M - Mc) : 0.0f, f2 = L2 > 0.0f ? fast_exp2(M2 - Mc) : 0.0f;
+      L = L * f1 + (f2 > 0.0f ? L2 * f2 : 0.0f);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        oh[i] = oh[i] * f1 + e[(2 + i) * 256] * f2;
+        orc[i] = orc[i] * f1 + e[(6 + i) * 256] * f2;
+      }
+    }
+    __syncthreads();
+  }
+  if (part != 0 || row >= rule.rows) return;
+  const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+  const int t = row / g, j = row - t * g;
+  const int64_t oi = (((int64_t)b * p.q_len + t) * p.n_q_heads + (int64_t)h * g + j) * 128 + d;
+  float o[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    o[i] = oh[i] * inv;
+    // history and recent outputs each in the output dtype, then added
+    if (rule.n_recent > 0) o[i] = round_out(p, round_out(p, o[i]) + round_out(p, orc[i] * inv));
+    o[i] = poisoned ? kQuietNaN : o[i];
+  }
+  store_out2(p, oi, o[0], o[1]);
+  store_out2(p, oi + 2, o[2], o[3]);
+}
+
+// The units of a (sequence, KV head) with several row tiles, merged by one
+// workgroup each (the shares as attn_rows_kernel computes them).
+__global__ __launch_bounds__(256) void rows_combine_kernel(smaq_attn_params p, RowsRule rule, int step,
+                                                           const float* __restrict__ slots, Partials recent);
+
 template <int KEY, int VB, typename TN, typename TV>
 __global__ __launch_bounds__(RowsKey<KEY>::kWaves * 64)
     __attribute__((amdgpu_waves_per_eu(kRowsPerSimd, kRowsPerSimd))) void attn_rows_kernel(
@@ -167,35 +320,16 @@ __global__ __launch_bounds__(RowsKey<KEY>::kWaves * 64)
 
   // ---- this workgroup's share [x, x_end) of the steps
   const uint32_t per_seq = (uint32_t)(p.n_kv_heads * rule.tiles);  // units per sequence
-  auto steps_of = [&](int64_t len) -> uint32_t { return len > 0 ? (uint32_t)((len + kStep - 1) / kStep) : 1u; };
+  auto steps_of = [&](int64_t len) -> uint32_t { return rows_steps(len, (int)kStep); };
   auto length_of = [&](int b) -> int64_t {
     return uniform64(p.hist_len ? min(max(((ConstI64Ptr)p.hist_len)[b], (int64_t)0), (int64_t)p.max_hist_len)
                                 : (int64_t)p.max_hist_len);
   };
-  uint32_t total;
-  if (p.hist_len) {
-    uint32_t sum = 0;
-    for (int b0 = 0; b0 < p.batch; b0 += 64) {
-      const int b = b0 + lane;
-      if (b < p.batch) sum += steps_of(min((int64_t)p.hist_len[b], (int64_t)p.max_hist_len));
-    }
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) sum += (uint32_t)__shfl_xor((int)sum, o, 64);
-    total = (uint32_t)__builtin_amdgcn_readfirstlane(sum) * per_seq;
-  } else {
-    total = steps_of(p.max_hist_len) * (uint32_t)p.batch * per_seq;
-  }
-  const uint32_t G = min((uint32_t)rule.groups, (total + rule.least - 1) / rule.least);
-  if ((uint32_t)wg >= G) return;
-  // the first `more` shares hold each + 1 steps, the others `each`
-  const uint32_t each = (uint32_t)__builtin_amdgcn_readfirstlane(total / G), more = total - each * G;
-  uint32_t x = (uint32_t)wg * each + min((uint32_t)wg, more);
-  const uint32_t x_end = x + each + ((uint32_t)wg < more ? 1u : 0u);
-  // the workgroup whose share holds step y
-  auto owner = [&](uint32_t y) -> uint32_t {
-    const uint32_t low = more * (each + 1);
-    return y < low ? y / (each + 1) : more + (y - low) / each;
-  };
+  const RowsShares share = rows_shares(p, rule, (int)kStep, lane);
+  if ((uint32_t)wg >= share.groups) return;
+  uint32_t x = share.start((uint32_t)wg);
+  const uint32_t x_end = share.start((uint32_t)wg + 1);
+  auto owner = [&](uint32_t y) -> uint32_t { return share.owner(y); };
   // the sequence of step x, and the steps before it
   int b = 0;
   uint32_t x_seq = 0;  // first step of sequence b
@@ -672,7 +806,7 @@ __global__ __launch_bounds__(RowsKey<KEY>::kWaves * 64)
       zacc[gg] += __shfl_xor(zacc[gg], 32, 64);
     }
     const uint32_t w_first = owner(x_unit), w_last = owner(x_unit + steps - 1);
-    const bool direct = rule.tiles == 1 && w_first == w_last && rule.n_recent == 0;
+    const bool direct = w_first == w_last && rule.n_recent == 0;
     float* const slot = slots + (int64_t)((uint32_t)wg + unit) * kRowsSlot;
     if (lane < kRowsQ) {
       red_m[wu][lane] = mref;
@@ -734,17 +868,17 @@ __global__ __launch_bounds__(RowsKey<KEY>::kWaves * 64)
     __syncthreads();  // red_o and red_l before the next unit's tiles
     if (direct) continue;
 
-    // ---- merge: the last piece of a (sequence, KV head) to arrive merges
-    // its units in piece order (the arrival protocol of attention_mfma.hip)
+    // ---- merge: the last piece of a unit to arrive merges it in piece order
+    // (the arrival protocol of attention_mfma.hip; the counters are per
+    // (sequence, KV head), so several units of one are merged by a launch of
+    // their own)
+    if (rule.tiles > 1) continue;
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(kWaitVmemOnly);
     asm volatile("" ::: "memory");
     __syncthreads();
-    const uint32_t x_head = x_unit - (uint32_t)rt * steps;  // first step of the head's units
     if (tid == 0) {
-      int pieces = 0;
-      for (int i = 0; i < rule.tiles; ++i)
-        pieces += (int)(owner(x_head + (uint32_t)(i + 1) * steps - 1) - owner(x_head + (uint32_t)i * steps)) + 1;
+      const int pieces = (int)(w_last - w_first) + 1;
       int* const cnt = p.arrivals + ((int64_t)b * p.n_kv_heads + h);
       const int before = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       const int last = before == pieces - 1 ? 1 : 0;
@@ -755,114 +889,8 @@ __global__ __launch_bounds__(RowsKey<KEY>::kWaves * 64)
     const bool merging = flag != 0;
     __syncthreads();  // flag is read before the next unit writes it
     if (!merging) continue;
-    // 256 threads take a tile's 8 rows x 32 dim quads; with 512, the two
-    // halves take alternate pieces.  A merge is a chain of memory round
-    // trips, so each has many loads in flight.
-    constexpr int kParts = kThreads / 256, kDeep = 8;
-    float* const ex = (float*)&vsp[0][0];  // the second half's sums
-    static_assert(kParts == 1 || sizeof(vsp) >= 256 * 11 * sizeof(float), "merge exchange");
-    const int part = tid >> 8, r = (tid & 255) >> 5, d = 4 * (tid & 31);
-    for (int ti = 0; ti < rule.tiles; ++ti) {
-      const uint32_t xu = x_head + (uint32_t)ti * steps;
-      const uint32_t w0 = owner(xu), w1 = owner(xu + steps - 1);
-      const uint32_t s_first = w0 + (uint32_t)b * per_seq + (uint32_t)(h * rule.tiles + ti);
-      const auto rs = __builtin_amdgcn_make_buffer_rsrc(slots + (int64_t)s_first * kRowsSlot, (short)0, -1, 0x00020000);
-      const int row = ti * kRowsQ + r, np = (int)(w1 - w0) + 1, n_all = np + rule.n_recent;
-      const int64_t rbase =
-          rule.n_recent > 0 ? recent.idx(b, h, p.n_kv_heads, rule.rows, min(row, rule.rows - 1), 0) : 0;
-      float M = -__builtin_inff(), L = 0.0f;
-      f32x4 oh = {0.0f, 0.0f, 0.0f, 0.0f}, orc = oh;
-      bool poisoned = false;  // a partial's sum is NaN
-      for (int c0 = part; c0 < n_all; c0 += kParts * kDeep) {
-        float mv[kDeep], lv[kDeep];
-        f32x4 ov[kDeep];
-#pragma unroll
-        for (int k = 0; k < kDeep; ++k) {
-          const int c = c0 + k * kParts;
-          mv[k] = -__builtin_inff();
-          lv[k] = 0.0f;
-          ov[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-          if (c < np) {  // (agent-coherent: written through by the other workgroups)
-            const int off = c * kRowsSlot * 4;
-            mv[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, r * 4, off, kAgentPolicy));
-            lv[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, (kRowsQ + r) * 4, off, kAgentPolicy));
-            ov[k] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                        rs, (2 * kRowsQ + r * 128 + d) * 4, off, kAgentPolicy));
-          } else if (c < n_all) {  // the recent window's partials (natural-log maxima)
-            const int64_t ri = rbase + (c - np);
-            mv[k] = recent.m[ri] * kLog2e;
-            lv[k] = recent.l[ri];
-            ov[k] = *(const f32x4*)&recent.o[ri * 128 + d];
-          }
-        }
-        float Mc = M;
-#pragma unroll
-        for (int k = 0; k < kDeep; ++k) {
-          poisoned |= lv[k] != lv[k];
-          Mc = lv[k] > 0.0f ? fmaxf(Mc, mv[k]) : Mc;
-        }
-        const float c = M == -__builtin_inff() ? 0.0f : fast_exp2(M - Mc);
-        L *= c;
-        oh *= c;
-        orc *= c;
-        M = Mc;
-#pragma unroll
-        for (int k = 0; k < kDeep; ++k) {
-          const bool live = lv[k] > 0.0f;
-          const float wk = live ? fast_exp2(mv[k] - M) : 0.0f;
-          L = live ? fmaf(lv[k], wk, L) : L;
-          const bool hist = c0 + k * kParts < np;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float v = live ? ov[k][i] : 0.0f;
-            oh[i] = fmaf(v, hist ? wk : 0.0f, oh[i]);
-            orc[i] = fmaf(v, hist ? 0.0f : wk, orc[i]);
-          }
-        }
-      }
-      if constexpr (kParts == 2) {
-        __syncthreads();
-        float* const e = ex + (tid & 255);
-        if (part == 1) {
-          e[0] = L;
-          ((uint32_t*)e)[10 * 256] = poisoned ? 1u : 0u;
-          e[256] = M;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            e[(2 + i) * 256] = oh[i];
-            e[(6 + i) * 256] = orc[i];
-          }
-        }
-        __syncthreads();
-        if (part == 0) {
-          const float L2 = e[0], M2 = e[256];
-          poisoned |= ((const uint32_t*)e)[10 * 256] != 0u;
-          const float Mc = fmaxf(M, M2);
-          const float f1 = L > 0.0f ? fast_exp2(M - Mc) : 0.0f, f2 = L2 > 0.0f ? fast_exp2(M2 - Mc) : 0.0f;
-          L = L * f1 + (f2 > 0.0f ? L2 * f2 : 0.0f);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            oh[i] = oh[i] * f1 + e[(2 + i) * 256] * f2;
-            orc[i] = orc[i] * f1 + e[(6 + i) * 256] * f2;
-          }
-        }
-        __syncthreads();
-      }
-      if (part != 0 || row >= rule.rows) continue;
-      const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-      const int t = row / g, j = row - t * g;
-      const int64_t oi = (((int64_t)b * p.q_len + t) * p.n_q_heads + (int64_t)h * g + j) * 128 + d;
-      float o[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        o[i] = oh[i] * inv;
-        // history and recent outputs each in the output dtype, then added
-        if (rule.n_recent > 0) o[i] = round_out(p, round_out(p, o[i]) + round_out(p, orc[i] * inv));
-        o[i] = poisoned ? kQuietNaN : o[i];
-      }
-      store_out2(p, oi, o[0], o[1]);
-      store_out2(p, oi + 2, o[2], o[3]);
-    }
+    rows_merge<kThreads / 256>(p, rule, recent, slots + (int64_t)(w_first + unit) * kRowsSlot, (int)(w_last - w_first) + 1,
+                               b, h, 0, tid, (float*)&vsp[0][0]);
     __syncthreads();  // (a later unit writes vsp)
   }
 }

@@ -7,10 +7,27 @@ namespace smaq {
 void launch_rows_vq(const smaq_attn_params& p, const HistAddr& a, const RowsRule& rule, float* slots,
                     const Partials& recent, hipStream_t st);
 
+__global__ __launch_bounds__(256) void rows_combine_kernel(smaq_attn_params p, RowsRule rule, int step,
+                                                           const float* __restrict__ slots, Partials recent) {
+  const int ti = blockIdx.x, h = blockIdx.y, b = blockIdx.z, tid = threadIdx.x, lane = tid & 63;
+  const RowsShares share = rows_shares(p, rule, step, lane);
+  const uint32_t units = (uint32_t)(p.n_kv_heads * rule.tiles), u = (uint32_t)(h * rule.tiles + ti);
+  const int64_t len = p.hist_len ? min((int64_t)p.hist_len[b], (int64_t)p.max_hist_len) : (int64_t)p.max_hist_len;
+  const uint32_t steps = rows_steps(len, step);
+  const uint32_t x = rows_sum_steps(p, step, b, lane) * units + u * steps;
+  const uint32_t w0 = share.owner(x), w1 = share.owner(x + steps - 1);
+  if (w0 == w1 && rule.n_recent == 0) return;  // written by its workgroup
+  rows_merge<1>(p, rule, recent, slots + (int64_t)(w0 + (uint32_t)b * units + u) * kRowsSlot, (int)(w1 - w0) + 1, b, h,
+                ti, tid, nullptr);
+}
+
+// query tokens below the prefill kernel's own range
+constexpr int kRowsMaxT = 63;
+
 bool rows_supported(const smaq_attn_params& p) {
   const bool known = p.val_dtype == SMAQ_F32 || p.val_dtype == SMAQ_F16 || p.val_dtype == SMAQ_BF16;
   if (p.impl != 0 || !p.has_history || p.max_hist_len <= 0 || !p.arrivals || p.head_dim != 128 || !known) return false;
-  if (p.q_len >= 16 || p.val_group != 32) return false;
+  if (p.q_len > kRowsMaxT || p.val_group != 32 || p.n_kv_heads > 65535 || p.batch > 65535) return false;
   if (!(p.val_bits == 2 && p.val_row_bytes == 32) && !(p.val_bits == 4 && p.val_row_bytes == 64)) return false;
   uintptr_t loads = (uintptr_t)p.val_bytes | (uintptr_t)p.q_hist | (uintptr_t)p.key_bytes | (uintptr_t)p.workspace;
   if (p.key_format == SMAQ_KEY_SCALAR) {
@@ -27,6 +44,22 @@ bool rows_supported(const smaq_attn_params& p) {
   if (units * ((double)p.max_hist_len / 128.0 + 1.0) > 1e9 || units > 1e6) return false;
   // (16-token halves of a tile lie in one page)
   return !p.block_table || (p.block_size >= 16 && (p.block_size & (p.block_size - 1)) == 0);
+}
+
+// From 16 query tokens on the prefill kernel serves the call as well.  It
+// decodes every key once into tile images and takes 256 query rows of one head
+// at a time, mostly empty ones for a short chunk; this kernel decodes a key
+// once per 8 rows.  Times over tokens x KV heads of history (MI355X, whole
+// plan): this kernel 25.5 ps per tile of 8 rows, prefill 0.46 ns and 0.22 ns
+// per query head, and about 20 us and 0.25 us per query token more beside
+// them.  30000 tokens (prefill / this kernel, us): 32/8 heads T = 16 373 / 80,
+// 32 372 / 123, 64 389 / 213, 128 427 / 386; 28/4 heads T = 32 318 / 114; 4000
+// tokens, 28/4 heads, T = 16 94 / 37, 32 98 / 48.  From kRowsMaxT tokens on the
+// choice is the prefill kernel's, as callers of such chunks know it.
+bool rows_preferred(const smaq_attn_params& p) {
+  const double g = p.n_q_heads / p.n_kv_heads, tiles = (double)((p.q_len * (p.n_q_heads / p.n_kv_heads) + kRowsQ - 1) / kRowsQ);
+  const double tokens = (double)p.batch * p.n_kv_heads * (double)p.max_hist_len;
+  return tokens * (0.0255 * tiles - 0.46 - 0.22 * g) * 1e-3 < 20.0 + 0.25 * p.q_len;
 }
 
 // Workgroups of the grid: what the device holds at once.
@@ -62,6 +95,11 @@ int launch_rows(const smaq_attn_params& p, const HistAddr& a, void* slots, const
       case SMAQ_F16: two ? launch_rows_v<0, 2, _Float16>(p, a, rule, s, recent, st) : launch_rows_v<0, 4, _Float16>(p, a, rule, s, recent, st); break;
       default: two ? launch_rows_v<0, 2, bf16>(p, a, rule, s, recent, st) : launch_rows_v<0, 4, bf16>(p, a, rule, s, recent, st); break;
     }
+  }
+  if (rule.tiles > 1) {
+    const int step = (p.key_format == SMAQ_KEY_SCALAR ? RowsKey<0>::kWaves : RowsKey<8>::kWaves) * kRowsTile;
+    hipLaunchKernelGGL(rows_combine_kernel, dim3((unsigned)rule.tiles, (unsigned)p.n_kv_heads, (unsigned)p.batch),
+                       dim3(256), 0, st, p, rule, step, s, recent);
   }
   return launch_status("smaq_attn_hybrid(rows)");
 }

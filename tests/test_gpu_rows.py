@@ -37,7 +37,7 @@ def _close(got, ref, vals, what):
 # (codec, key bits or block dim, value bits, heads per KV head, query tokens, storage dtype)
 FORMS = [("vq", 2, 2, 7, 1, torch.float16), ("vq", 4, 4, 8, 1, torch.bfloat16), ("vq", 8, 2, 4, 3, torch.bfloat16),
          ("vq", 8, 4, 1, 1, torch.float32), ("scalar", 3, 2, 7, 1, torch.bfloat16), ("scalar", 4, 4, 3, 1, torch.float16),
-         ("scalar", 3, 4, 2, 15, torch.float32), ("scalar", 4, 2, 16, 2, torch.float32)]
+         ("scalar", 3, 4, 2, 15, torch.float32), ("scalar", 4, 2, 16, 2, torch.float32), ("vq", 2, 4, 3, 63, torch.bfloat16)]
 
 
 @pytest.mark.parametrize("codec,size,vbits,g,T,dtype", FORMS)
@@ -46,7 +46,7 @@ def test_rows_store_edges(dev, codec, size, vbits, g, T, dtype):
     tokens and a share of several steps; with and without a recent window and
     a causal limit; a repeated call gives the same bits."""
     strat = _strategy(dev, codec, size)
-    for n, rn in ((16, 0), (33, 1), (127, 64), (257, 65), (513, 0), (2051, 128)):
+    for n, rn in ((63, 0) if T > 16 else (16, 0), (33, 31) if T > 16 else (33, 1), (127, 64), (257, 65), (513, 0), (2051, 128)):
         st = S.CompressedKVStore(128, 2, value_bits=vbits, device=dev, key_strategy=strat)
         k = sample_keys(n * 2, seed=n).view(n, 2, 128).to(dtype).to(dev)
         v = torch.randn(n, 2, 128, generator=torch.Generator().manual_seed(n)).to(dtype).to(dev)
