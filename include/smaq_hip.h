@@ -83,6 +83,35 @@ int smaq_apply_values(const float* w, long long w_bstride, long long w_qstride, 
                       void* workspace, long long workspace_bytes, void* stream);
 
 /*
+ * smaq_apply_values with the exact window's term of SMAQKVCache.attend
+ * (smaq/kv_cache.py:253-262) in the same call: weights w[b][q][N + r] times the
+ * R exact fp32 rows xv + b * xv_bstride + r * D are added.  D <= 256 when R > 0
+ * or a multiple of 256.
+ */
+long long smaq_cache_attend_workspace_bytes(long long batch, long long nq, long long N, long long R, int D);
+int smaq_cache_attend(const float* w, long long w_bstride, long long w_qstride, long long batch, long long nq,
+                      long long N, int D, const void* data, long long d_bstride, int bits, int group,
+                      const void* scales, const void* zeros, long long s_bstride, int sdtype, long long R,
+                      const float* xv, long long xv_bstride, float* out, void* workspace, long long workspace_bytes,
+                      void* stream);
+
+/*
+ * Scores of the standalone cache's decode step.  Replaces
+ * SMAQKVCache.attention_scores (smaq/kv_cache.py:218-241) for head_dim 128 and
+ * 3- or 4-bit scalar keys: out[b][r][0..N) = ((q M^T)[b][r] . c[code[b][t]]) *
+ * norm[b][t] * scale, out[b][r][N..N+R) = (q[b][r] . xk[b][t], rounded) * scale.
+ *   q [batch][nq][128] in qdtype; M [128][128] fp32 row-major (E_inv), 16-byte
+ *   aligned; qrot: batch * nq * 128 floats of workspace; code rows of 64 bytes
+ *   at codes + b * codes_bstride + 64 t (16-byte aligned), norms at
+ *   b * norm_bstride + t in ndtype; xk rows of 128 qdtype elements at
+ *   b * xk_bstride + 128 t; out [batch][nq][N + R] in qdtype.
+ */
+int smaq_cache_scores(const void* q, int qdtype, long long batch, long long nq, int D, const float* M, float* qrot,
+                      long long N, const void* codes, long long codes_bstride, int bits, const void* norms,
+                      long long norm_bstride, int ndtype, const float* centroids, long long R, const void* xk,
+                      long long xk_bstride, float scale, void* out, void* stream);
+
+/*
  * Scalar key encoder.  Replaces SMAQQuantizer.quantize (smaq/quantizer.py:138-145)
  * and RotationAdapter.quantize (smaq/weighted_scalar.py:347-355):
  * n = ||k|| (key dtype), u = k / (n + 1e-10) (key dtype), y = u @ M^T (fp32),

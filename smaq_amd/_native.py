@@ -91,6 +91,12 @@ _SIGS = {
     "smaq_apply_values_workspace_bytes": (c_ll, [c_ll, c_ll, c_ll, c_int]),
     "smaq_apply_values": (c_int, [c_void_p, c_ll, c_ll, c_ll, c_ll, c_ll, c_int, c_void_p, c_ll, c_int, c_int,
                                   c_void_p, c_void_p, c_ll, c_int, c_void_p, c_void_p, c_ll, c_void_p]),
+    "smaq_cache_attend_workspace_bytes": (c_ll, [c_ll, c_ll, c_ll, c_ll, c_int]),
+    "smaq_cache_attend": (c_int, [c_void_p, c_ll, c_ll, c_ll, c_ll, c_ll, c_int, c_void_p, c_ll, c_int, c_int,
+                                  c_void_p, c_void_p, c_ll, c_int, c_ll, c_void_p, c_ll, c_void_p, c_void_p, c_ll,
+                                  c_void_p]),
+    "smaq_cache_scores": (c_int, [c_void_p, c_int, c_ll, c_ll, c_int, c_void_p, c_void_p, c_ll, c_void_p, c_ll, c_int,
+                                  c_void_p, c_ll, c_int, c_void_p, c_ll, c_void_p, c_ll, c_float, c_void_p, c_void_p]),
 }
 
 # Size of the built-in workspace of smaq_attn_hybrid_noalloc
@@ -330,6 +336,48 @@ def apply_values(w: torch.Tensor, data: torch.Tensor, scales: torch.Tensor, zero
                                    bits, group_size, _ptr(s3), _ptr(z3), s3.stride(0), dtype_code(s3.dtype),
                                    _ptr(out), _ptr(ws), max(ws_bytes, 0), _stream(dev)),
            "smaq_apply_values")
+    return out
+
+
+# --------------------------------------------------- standalone cache step ---
+
+def cache_scores(query: torch.Tensor, M: torch.Tensor, centroids: torch.Tensor, bits: int, codes: torch.Tensor,
+                 norms: torch.Tensor, n: int, exact, start: int, r: int, scale: float) -> torch.Tensor:
+    """[compressed, exact] scores of query [*lead, nq, 128] over the first n
+    rows of the columns codes [lanes, capacity, 64] and norms [lanes, capacity]
+    and rows [start, start + r) of ``exact`` [*lead, capacity, 128] (None: r is
+    0): [*lead, nq, n + r] in the query's dtype, two launches."""
+    q = query.contiguous()
+    nq, D = q.shape[-2:]
+    lanes, dev = codes.shape[0], q.device
+    qrot = torch.empty(lanes * nq * D, dtype=torch.float32, device=dev)
+    out = torch.empty(*q.shape[:-1], n + r, dtype=q.dtype, device=dev)
+    xk = xs = 0
+    if r:
+        xk, xs = exact.data_ptr() + start * D * exact.element_size(), exact.shape[-2] * D
+    _check(lib().smaq_cache_scores(q.data_ptr(), _DTYPE_CODE[q.dtype], lanes, nq, D, M.data_ptr(), qrot.data_ptr(), n,
+                                   codes.data_ptr(), codes.stride(0), bits, norms.data_ptr(), norms.stride(0),
+                                   _DTYPE_CODE[norms.dtype], centroids.data_ptr(), r, xk, xs, scale, out.data_ptr(),
+                                   _stream(dev)), "smaq_cache_scores")
+    return out
+
+
+def cache_attend(w: torch.Tensor, data: torch.Tensor, scales: torch.Tensor, zeros: torch.Tensor, bits: int,
+                 group: int, n: int, exact, start: int, r: int, D: int) -> torch.Tensor:
+    """Contiguous fp32 weights w [*lead, nq, n + r] over the first n rows of the
+    packed columns [lanes, capacity, ...] and rows [start, start + r) of the fp32
+    ``exact`` [*lead, capacity, D]: [*lead, nq, D] fp32, two launches."""
+    nq, lanes, dev = w.shape[-2], data.shape[0], w.device
+    out = torch.empty(*w.shape[:-1], D, dtype=torch.float32, device=dev)
+    xv = xs = 0
+    if r:
+        xv, xs = exact.data_ptr() + start * D * 4, exact.shape[-2] * D
+    size = lib().smaq_cache_attend_workspace_bytes(lanes, nq, n, r, D)
+    ws = torch.empty(size, dtype=torch.uint8, device=dev) if size > 0 else None
+    _check(lib().smaq_cache_attend(w.data_ptr(), nq * (n + r), n + r, lanes, nq, n, D, data.data_ptr(), data.stride(0),
+                                   bits, group, scales.data_ptr(), zeros.data_ptr(), scales.stride(0),
+                                   _DTYPE_CODE[scales.dtype], r, xv, xs, out.data_ptr(), _ptr(ws), size,
+                                   _stream(dev)), "smaq_cache_attend")
     return out
 
 

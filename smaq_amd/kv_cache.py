@@ -25,10 +25,15 @@ from smaq_amd import _native
 from smaq_amd.calibration import IdentityCalibrationProvider
 from smaq_amd.columns import ColumnHistory, codec_kind
 from smaq_amd.core import CacheCapabilities, CalibrationProvider
-from smaq_amd.quantizer import default_device
+from smaq_amd.quantizer import SMAQQuantizer, default_device
 from smaq_amd.strategies import SMAQFullMetricScalarStrategy
 from smaq_amd.value_codec import (ValueQuantized, dequantize_values, quantize_values,  # noqa: F401
                                   unpack_values)
+
+
+def _differentiated(t: torch.Tensor) -> bool:
+    """Whether a gradient or a tangent may be asked of an op on t."""
+    return (t.requires_grad and torch.is_grad_enabled()) or torch.autograd.forward_ad._current_level >= 0
 
 
 class _ExactWindow:
@@ -209,11 +214,40 @@ class SMAQKVCache:
         if over > 0:
             self._compress(*self._exact.pop_front(over))
 
+    def _exact_rows(self, buf: Optional[torch.Tensor], dtype: torch.dtype) -> bool:
+        """Whether the exact window (if any) is rows of ``dtype`` that the
+        one-call step reads in place."""
+        return self._exact.size == 0 or (buf.dtype == dtype and buf.is_contiguous() and buf.shape[:-2] == self._lead
+                                         and buf.device == self._hist._bufs["v_data"].device and not buf.requires_grad)
+
+    def _one_call(self, query: torch.Tensor) -> bool:
+        """Whether ``attention_scores`` of this query is one native call: plain
+        scalar SMAQ keys of 3 or 4 bits at head_dim 128 in columns, and a plain
+        GPU query of the cache's leading shape and the exact window's dtype."""
+        h, s = self._hist, self.key_quantizer
+        if (h is None or not h.n or type(s) is not SMAQFullMetricScalarStrategy or type(s.quantizer) is not SMAQQuantizer
+                or type(query) is not torch.Tensor or not query.is_cuda or _differentiated(query)):
+            return False
+        qz, codes = s.quantizer, h._bufs["k_codes"]
+        return (query.dim() >= 2 and query.shape[-1] == self.head_dim == qz.dim == 128 and qz.bits in (3, 4)
+                and query.shape[:-2] == self._lead and query.numel() > 0 and query.device == codes.device
+                and query.dtype in (torch.float32, torch.float16, torch.bfloat16) and codes.shape[0] < 65536
+                and qz.E_inv.dtype == torch.float32 and qz.E_inv.is_contiguous() and qz.E_inv.device == codes.device
+                and qz.E_inv.data_ptr() % 16 == 0 and qz.centroids.dtype == torch.float32
+                and qz.centroids.is_contiguous() and qz.centroids.numel() == 1 << qz.bits
+                and self._exact_rows(self._exact.k, query.dtype))
+
     def attention_scores(self, query: torch.Tensor, scale: float | None = None) -> torch.Tensor:
         """[compressed, exact] scores along the key axis, no softmax
         (smaq/kv_cache.py:218-241)."""
         if scale is None:
             scale = 1.0 / math.sqrt(self.head_dim)
+        if self._one_call(query):
+            # both parts in one native call, straight from the columns
+            h, ex, qz = self._hist, self._exact, self.key_quantizer.quantizer
+            bufs = h._bufs
+            return _native.cache_scores(query, qz.E_inv, qz.centroids, qz.bits, bufs["k_codes"], bufs["k_norms"], h.n,
+                                        ex.k, ex.start, ex.size, float(scale))
         parts = []
         kq = self.key_quantized
         if kq is not None:
@@ -230,6 +264,16 @@ class SMAQKVCache:
     def attend(self, attn_weights: torch.Tensor) -> torch.Tensor:
         """Weights over [compressed, exact] applied to the dequantised and the
         exact values (smaq/kv_cache.py:243-267)."""
+        h, ex = self._hist, self._exact
+        if (h is not None and h.n and type(attn_weights) is torch.Tensor and attn_weights.is_cuda
+                and attn_weights.dtype == torch.float32 and attn_weights.is_contiguous()
+                and attn_weights.device == h._bufs["v_data"].device and attn_weights.shape[:-2] == self._lead
+                and attn_weights.shape[-1] == h.n + ex.size and attn_weights.numel() and not _differentiated(attn_weights)
+                and self.head_dim in (32, 64, 128, 256) and self._exact_rows(ex.v, torch.float32)
+                and _native.apply_values_supported(self.head_dim, self.value_bits, self.value_group_size)):
+            bufs = h._bufs
+            return _native.cache_attend(attn_weights, bufs["v_data"], bufs["v_scales"], bufs["v_zeros"], self.value_bits,
+                                        self.value_group_size, h.n, ex.v, ex.start, ex.size, self.head_dim)
         out = None
         col = 0
         vq = self.value_quantized

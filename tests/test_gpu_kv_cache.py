@@ -143,3 +143,35 @@ def test_apply_values_matches_dequantized_matmul(dev, bits, group, sdtype, N):
     err = (got.double() - ref).abs()
     assert bool((err <= 2e-3 + 1e-3 * ref.abs()).all()), float(err.max())
     assert float(err.max()) <= 1e-5 * max(1.0, float(ref.abs().max())), float(err.max())
+
+
+@pytest.mark.parametrize("bits,vbits,dtype,lead,nq,total,buf", [
+    (3, 2, torch.float32, (2, 4), 1, 1000, 128), (4, 4, torch.float32, (3,), 5, 257 + 31, 31),
+    (3, 2, torch.float32, (), 4, 33, 32), (4, 2, torch.bfloat16, (1, 2), 3, 600, 17), (3, 8, torch.float16, (2, 1), 2, 300, 299),
+    (3, 2, torch.float32, (2, 2), 2, 515, 0)])
+def test_kv_cache_one_call_matches_the_general_path(dev, bits, vbits, dtype, lead, nq, total, buf):
+    """The one-call scores and attend against the general path, which a tensor
+    that requires a gradient takes: one exact token to all but one, window
+    positions after appends, several query rows.  Scores: the compressed ones
+    are the same bits; an exact one is a 128-term fp32 sum either way (within
+    2^-17 of its terms' magnitude, at most 30 here, and one output unit).
+    Attended rows: fp32 sums of one order or another, 2e-5 of the largest."""
+    cache = S.SMAQKVCache(128, key_bits=bits, value_bits=vbits, buffer_size=buf, device=dev)
+    cut = total - 5
+    k = sample_keys(total * max(1, int(torch.tensor(lead).prod())), seed=total).view(*lead, total, 128).to(dtype).to(dev)
+    v = torch.randn(*lead, total, 128, generator=torch.Generator().manual_seed(total)).to(dtype).to(dev)
+    cache.prefill(k[..., :cut, :], v[..., :cut, :])
+    for t in range(cut, total):
+        cache.append(k[..., t:t + 1, :], v[..., t:t + 1, :])
+    q = sample_keys(nq * max(1, int(torch.tensor(lead).prod())), seed=total + 1).view(*lead, nq, 128).to(dtype).to(dev)
+    assert cache._one_call(q) and not cache._one_call(q.clone().requires_grad_())
+    got, want = cache.attention_scores(q), cache.attention_scores(q.clone().requires_grad_()).detach()
+    n = total - cache._exact.size
+    assert got.shape == want.shape and got.dtype == want.dtype and torch.equal(got[..., :n], want[..., :n])
+    unit = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dtype]
+    err = (got[..., n:].float() - want[..., n:].float()).abs()
+    assert bool((err <= 30 * 2.0 ** -17 + 2 * unit * want[..., n:].float().abs()).all())
+    if dtype == torch.float32:
+        w = torch.softmax(got, dim=-1)
+        a, b = cache.attend(w), cache.attend(w.clone().requires_grad_()).detach()
+        assert a.shape == b.shape and float((a - b).abs().max()) <= 2e-5 * float(b.abs().max())
