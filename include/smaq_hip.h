@@ -313,7 +313,11 @@ typedef struct smaq_attn_params {
      phases 8 and 1 run in one call); with 16 added,
      phase 1 reuses the schedule an earlier call on this workspace built for
      the same lengths, so the decode kernel can be timed alone (with any
-     other workspace contents the output is undefined). */
+     other workspace contents the output is undefined).  32 added to the
+     phases wanted: q_raw is first written to q_exact as fp32 (by the recent
+     window's kernel when that one runs first, else by one launch), so a
+     caller with rot_mt NULL and q_hist = q_exact hands in the query as it
+     has it. */
   int phases;
   /* kernel choice: 0 = automatic (matrix-core decode kernel when the shape
      allows, generic kernels otherwise), 1 = generic kernels only, 2 = the

@@ -646,6 +646,11 @@ extern "C" int smaq_attn_hybrid(const smaq_attn_params* pp, void* stream) {
     SMAQ_REQUIRE((p.q_exact || p.q_raw) && p.recent_k && p.recent_v && p.max_recent_len > 0,
                  "smaq_attn_hybrid: null recent pointer");
   }
+  if (p.phases & 32) {
+    SMAQ_REQUIRE(p.q_raw && p.q_exact, "smaq_attn_hybrid: phase 32 without q_raw or q_exact");
+    SMAQ_REQUIRE(p.q_raw_dtype == SMAQ_F32 || p.q_raw_dtype == SMAQ_F16 || p.q_raw_dtype == SMAQ_BF16,
+                 "smaq_attn_hybrid: unsupported q_raw dtype %d", p.q_raw_dtype);
+  }
   Plan pl = make_plan(&p, true);
   // (a caller that sized its workspace before it set the arrival counters
   // has room for the generic kernels only)
@@ -699,6 +704,26 @@ extern "C" int smaq_attn_hybrid(const smaq_attn_params* pp, void* stream) {
   // the history phase (phase 8); when the recent window goes first as well
   // (and has the decode kernel), one launch runs both side by side.
   const bool rotation = p.has_history && p.rot_mt && (phases & 8);
+  // Phase 32, the raw query widened into q_exact: by the recent window's
+  // kernel, which stages those rows anyway, when it runs before whatever
+  // reads them; else by a launch of its own.
+  auto widen = [&]() -> int {
+    const int64_t n = (int64_t)p.batch * p.q_len * p.n_q_heads * p.head_dim;
+    const unsigned blocks = (unsigned)((n + 255) / 256);
+    switch (p.q_raw_dtype) {
+      case SMAQ_F32: hipLaunchKernelGGL(widen_kernel<float>, dim3(blocks), dim3(256), 0, st, (const float*)p.q_raw, n, (float*)p.q_exact); break;
+      case SMAQ_F16: hipLaunchKernelGGL(widen_kernel<_Float16>, dim3(blocks), dim3(256), 0, st, (const _Float16*)p.q_raw, n, (float*)p.q_exact); break;
+      default: hipLaunchKernelGGL(widen_kernel<bf16>, dim3(blocks), dim3(256), 0, st, (const bf16*)p.q_raw, n, (float*)p.q_exact); break;
+    }
+    return launch_status("smaq_attn_hybrid(query widen)");
+  };
+  const bool widened_by_recent =
+      !pl.prefill && pl.s_recent > 0 && recent_decode_supported(p) &&
+      (recent_first || ((phases & 2) && (pl.s_hist == 0 || !(phases & 1))));
+  if ((phases & 32) && !widened_by_recent) {
+    const int rc = widen();
+    if (rc != SMAQ_OK) return rc;
+  }
   const bool paired = recent_first && rotation && !pl.prefill && rotate_recent_supported(p);
   if (paired) {
     const int rc = launch_rotate_recent(p, part, pl.s_hist, pl.s_recent, pl.recent_split, st);
@@ -743,16 +768,9 @@ extern "C" int smaq_attn_hybrid(const smaq_attn_params* pp, void* stream) {
     if (pl.s_recent > 0 && (phases & 2)) {
       // the prefill kernel reads the plain query as fp32 rows: with a raw
       // query handed in, the library writes them into q_exact first
-      if (p.q_raw) {
+      if (p.q_raw && !(phases & 32)) {
         SMAQ_REQUIRE(p.q_exact, "smaq_attn_hybrid: the prefill recent part needs a q_exact buffer");
-        const int64_t n = (int64_t)p.batch * p.q_len * p.n_q_heads * p.head_dim;
-        const unsigned blocks = (unsigned)((n + 255) / 256);
-        switch (p.q_raw_dtype) {
-          case SMAQ_F32: hipLaunchKernelGGL(widen_kernel<float>, dim3(blocks), dim3(256), 0, st, (const float*)p.q_raw, n, (float*)p.q_exact); break;
-          case SMAQ_F16: hipLaunchKernelGGL(widen_kernel<_Float16>, dim3(blocks), dim3(256), 0, st, (const _Float16*)p.q_raw, n, (float*)p.q_exact); break;
-          default: hipLaunchKernelGGL(widen_kernel<bf16>, dim3(blocks), dim3(256), 0, st, (const bf16*)p.q_raw, n, (float*)p.q_exact); break;
-        }
-        int rc = launch_status("smaq_attn_hybrid(query widen)");
+        const int rc = widen();
         if (rc != SMAQ_OK) return rc;
       }
       int rc = launch_prefill_planes_recent(p, rp, st);

@@ -138,8 +138,15 @@ __device__ __forceinline__ void recent_block(RecentLds<G>& L, const smaq_attn_pa
   const int64_t t1 = min(len, t0 + split_len);
 
   // the G query rows of this tile, staged in LDS (lane (tq, dq) reads
-  // dims 32 dq .. of each)
-  for (int i = tid; i < G * kRD; i += 256) qs[i / kRD][i % kRD] = exact_query(p, row_off(i / kRD) + i % kRD);
+  // dims 32 dq .. of each); phase 32: the first split writes them to q_exact
+  const bool keep = (p.phases & 32) && s == 0;
+  for (int i = tid; i < G * kRD; i += 256) {
+    const int g = i / kRD, d = i % kRD;
+    const int64_t at = row_off(g) + d;
+    const float x = exact_query(p, at);
+    qs[g][d] = x;
+    if (keep && g < nr) const_cast<float*>(p.q_exact)[at] = x;
+  }
   if (tid < G) {
     m_s[tid] = -__builtin_inff();
     l_s[tid] = 0.0f;

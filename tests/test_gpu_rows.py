@@ -130,3 +130,30 @@ def test_rows_small_workspace_runs_generic(dev):
     assert small < plan.params.workspace_bytes
     plan.params.workspace_bytes = small
     assert torch.equal(plan.run(q).view_as(want), want)
+
+
+@pytest.mark.parametrize("T,rn,impl,dtype", [(1, 0, 0, torch.bfloat16), (1, 70, 0, torch.float16), (3, 129, 0, torch.bfloat16),
+                                             (63, 5, 0, torch.float32), (1, 70, 1, torch.bfloat16),
+                                             (64, 40, 3, torch.bfloat16), (64, 0, 0, torch.float16)])
+def test_unrotated_query_is_widened_by_the_library(dev, T, rn, impl, dtype):
+    """A run of an unrotated codec's plan gives the bits of a loaded query and
+    a launch, leaves the fp32 query in q_exact for a later launch, and keeps
+    no pointer to the caller's query; a strided query still runs."""
+    n, g = 300, 3
+    k = sample_keys(2 * n * 2, seed=1).view(2, n, 2, 128).to(dev)
+    v = torch.randn(2, n, 2, 128, generator=torch.Generator().manual_seed(2)).to(dev)
+    kvb = QuantizedKVBatch.encode(_strategy(dev, "vq", 8), k, v)
+    q = sample_keys(2 * T * 2 * g, seed=3).view(2, T, 2 * g, 128).to(dtype).to(dev)
+    rk = sample_keys(2 * rn * 2, seed=4).view(2, rn, 2, 128).bfloat16().to(dev) if rn else None
+    plan = kvb.plan(q, None, rk, rk, torch.tensor([0, rn], device=dev) if rn else None, impl)
+    plan.load_query(q)
+    ref = plan.launch().clone()
+    plan.q_exact.fill_(float("nan"))
+    assert torch.equal(plan.run(q), ref) and torch.equal(plan.q_exact, q.float())
+    assert plan.params.q_raw is None and plan.params.phases == 0
+    assert torch.equal(plan.launch(), ref)
+    strided = torch.stack([q, q + 1], dim=-1)[..., 0]
+    plan.q_exact.fill_(float("nan"))
+    assert torch.equal(plan.run_into(strided, torch.empty_like(plan.out)), ref)
+    plan.q_exact.fill_(float("nan"))
+    assert torch.equal(plan.run_into(q, torch.empty_like(plan.out)), ref)
