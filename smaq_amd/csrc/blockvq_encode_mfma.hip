@@ -31,14 +31,19 @@
 // are the columns of four MFMA products per codebook tile, which share the
 // tile's one LDS read, and the key blocks of the next block are in flight
 // meanwhile.  Each lane keeps, per
-// group, the running minimum of its 64 distances as the distance bits with
-// the low 8 bits replaced by the centroid's position in the lane (tile, row),
-// so one v_min3_u32 tracks value and index of two distances (distances are
-// positive: delta is added to every one) and a v_med3_u32 / v_min_u32 pair the
-// runner-up.  The four k-group lanes of every token are then merged by
-// v_permlane32_swap / v_permlane16_swap reduce-scatters (the k-group goes into
-// tag bits 7:6), leaving token l of the set in lane l for the clear test, the
-// index, the store and the exact recount.
+// group, the nearest and second nearest of its 16 quads of centroids (a
+// product's four rows), as the bits of the quad's smallest distance with the
+// low 6 bits replaced by the quad's position (tile, k-group): distances are
+// positive (delta is added to every one), so a v_min and a v_min3_u32 reduce a
+// quad, and one v_min3_u32 and a v_med3_u32 / v_min_u32 pair keep two quads'
+// value, index and runner-up.  The four k-group lanes of every token are then
+// merged by v_permlane32_swap / v_permlane16_swap reduce-scatters, leaving
+// token l of the set in lane l, which forms the nearest quad's four distances
+// again from the LDS codebook (the same terms, v_dot2_f32_f16: at most 2^-23 S
+// for each of 13 steps, 1.6e-6) for the clear test, the index, the store and
+// the exact recount.  VALU bound (81 % of the cycles of 16 waves per CU); value
+// and index of every single distance took 30 % more VALU instructions:
+// 4,194,304 rows of 16 blocks, their value pack included, 2253 -> 2116 us.
 #include "encode_internal.h"
 
 namespace smaq {
@@ -47,6 +52,7 @@ namespace {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kVmWaves = 16;                  // waves per workgroup (4 per SIMD)
 constexpr int kVmThreads = 64 * kVmWaves;
@@ -76,6 +82,10 @@ __device__ __forceinline__ uint32_t fbits(float x) { return __builtin_bit_cast(u
 __device__ __forceinline__ float bitsf(uint32_t b) { return __builtin_bit_cast(float, b); }
 __device__ __forceinline__ uint32_t h16(_Float16 h) { return (uint32_t)__builtin_bit_cast(uint16_t, h); }
 
+// a + x . y of two f16 pairs
+__device__ __forceinline__ float dot2(uint32_t x, uint32_t y, float a) {
+  return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, x), __builtin_bit_cast(f16x2, y), a, false);
+}
 // Two keys k0, k1 at a time: with best <= second, the new minimum is
 // min3(best, k0, k1) and the new runner-up min(second, med3(best, k0, k1))
 // (the overall minimum lies in {best, k0, k1}, so the second smallest of the
@@ -109,6 +119,17 @@ __device__ __forceinline__ float reduce_scatter_kgroups(const float* v) {
   const float s13 = bitsf(q[0]) + bitsf(q[1]);  // rows 0-1: token (1, n), rows 2-3: (3, n)
   const auto r = __builtin_amdgcn_permlane16_swap(fbits(s02), fbits(s13), false, false);
   return bitsf(r[0]) + bitsf(r[1]);
+}
+// The four k-groups' values of token (r, n), to lane (r, n).
+__device__ __forceinline__ void transpose_kgroups(const uint32_t* v, uint32_t* out) {
+  const auto p = __builtin_amdgcn_permlane32_swap(v[0], v[2], false, false);
+  const auto q = __builtin_amdgcn_permlane32_swap(v[1], v[3], false, false);
+  const auto a = __builtin_amdgcn_permlane16_swap(p[0], q[0], false, false);
+  const auto b = __builtin_amdgcn_permlane16_swap(p[1], q[1], false, false);
+  out[0] = a[0];
+  out[1] = a[1];
+  out[2] = b[0];
+  out[3] = b[1];
 }
 // The inverse direction: x of lane (r, n) belongs to token (r, n); every lane
 // of column n receives out[g] = x of token (g, n).
@@ -328,7 +349,7 @@ __global__ __launch_bounds__(kVmThreads) void encode_blockvq_mfma_kernel(
     kp[g] = key_row(set, g);
     kb[g].load(kp[g]);
   }
-  const uint32_t kg_tag = (uint32_t)kg << 6;
+  const uint32_t kg_tag = (uint32_t)kg << 4;
   for (; set < n_sets; set += stride) {
     const int64_t row = set * 64 + lane;  // the token this lane finishes
     const bool valid = row < rows;
@@ -348,6 +369,7 @@ __global__ __launch_bounds__(kVmThreads) void encode_blockvq_mfma_kernel(
       // ---- the four groups' B operands (staged one group at a time through
       // the wave's 16-token buffer) and C operands sigma^2 (|x|^2 + delta)
       f16x8 bv[4];
+      uint32_t yh[4], yl[4];  // y hi, lo of dims kg, kg + 4 of token (g, n)
       float sqp[4];  // this k-group's part of |x|^2 of token (g, n)
       // the key blocks loaded next: block b + 1 of these tokens, or block 0
       // of the next set's
@@ -373,8 +395,10 @@ __global__ __launch_bounds__(kVmThreads) void encode_blockvq_mfma_kernel(
         const bool ok = fabsf(ya) < kYMax && fabsf(yb) < kYMax;  // false for NaN
         const _Float16 yah = (_Float16)ya, ybh = (_Float16)yb;
         const _Float16 yal = (_Float16)(ya - (float)yah), ybl = (_Float16)(yb - (float)ybh);
-        *(__attribute__((address_space(3))) uint32_t*)(lds3 + ys_tok + 4 * kg) = h16(yah) | (h16(ybh) << 16);
-        *(__attribute__((address_space(3))) uint32_t*)(lds3 + ys_tok + 16 + 4 * kg) = h16(yal) | (h16(ybl) << 16);
+        yh[g] = h16(yah) | (h16(ybh) << 16);
+        yl[g] = h16(yal) | (h16(ybl) << 16);
+        *(__attribute__((address_space(3))) uint32_t*)(lds3 + ys_tok + 4 * kg) = yh[g];
+        *(__attribute__((address_space(3))) uint32_t*)(lds3 + ys_tok + 16 + 4 * kg) = yl[g];
         sqp[g] = ok ? xa * xa + xb * xb : __builtin_nanf("");
         wave_sync();
         // B: k-group 0 / 2 take y hi, 1 takes y lo, 3 the 2^14 pair of block b
@@ -390,7 +414,8 @@ __global__ __launch_bounds__(kVmThreads) void encode_blockvq_mfma_kernel(
       const float delta = kDeltaRel * (sq + smax_b);
       const float delta_s = delta * s2;
       float init_g[4];
-      all_gather_kgroups((sq + delta) * s2, init_g);
+      const float init = (sq + delta) * s2;
+      all_gather_kgroups(init, init_g);
       f32x4 cv[4];
 #pragma unroll
       for (int g = 0; g < 4; ++g) cv[g] = f32x4{init_g[g], init_g[g], init_g[g], init_g[g]};
@@ -398,7 +423,7 @@ __global__ __launch_bounds__(kVmThreads) void encode_blockvq_mfma_kernel(
       // the next (tile, group) issued before the keys of this one are reduced
       const LdsU32x4* ap =
           (LdsU32x4*)(lds3 + a_src + (kg < 3 ? (uint32_t)b * a_blk : (uint32_t)(b >> 2) * (uint32_t)(kVmNc * 16)));
-      uint32_t best[4], second[4];
+      uint32_t best[4], second[4], even[4];
 #pragma unroll
       for (int g = 0; g < 4; ++g) best[g] = second[g] = 0xffffffffu;
       u32x4 a_cur = ap[0], a_nxt = ap[16];
@@ -415,14 +440,16 @@ __global__ __launch_bounds__(kVmThreads) void encode_blockvq_mfma_kernel(
           }
           acc_next = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a_cur), bv[g1], cv[g1], 0, 0, 0);
         }
-#pragma unroll
-        for (int i = 0; i < 4; i += 2) {
-          // centroids 16t + 4kg + i, i + 1 of token (g, n); low 8 bits =
-          // (0, t, i) now, the k-group goes into bits 6-7 below
-          const uint32_t k0 = (fbits(acc[i]) & 0xffffff00u) | (uint32_t)(4 * t + i);
-          const uint32_t k1 = (fbits(acc[i + 1]) & 0xffffff00u) | (uint32_t)(4 * t + i + 1);
-          second[g] = min(second[g], med3_u32(best[g], k0, k1));
-          best[g] = min3_u32(best[g], k0, k1);
+        // the nearest of centroids 16t + 4kg .. + 3 of token (g, n); low 6 bits
+        // = (0, t) now, the k-group goes into bits 4-5 below
+        // (not min3_u32: the compiler does not wait for a product read by asm)
+        const uint32_t m = min(min(min(fbits(acc[0]), fbits(acc[1])), fbits(acc[2])), fbits(acc[3]));
+        const uint32_t key = (m & 0xffffffc0u) | (uint32_t)t;
+        if (t & 1) {
+          second[g] = min(second[g], med3_u32(best[g], even[g], key));
+          best[g] = min3_u32(best[g], even[g], key);
+        } else {
+          even[g] = key;
         }
       }
       // ---- merge the four k-group lanes of every token, leaving token
@@ -444,14 +471,43 @@ __global__ __launch_bounds__(kVmThreads) void encode_blockvq_mfma_kernel(
       const auto ps = __builtin_amdgcn_permlane16_swap(ms[0], ms[1], false, false);
       const uint32_t gbest = min(pb[0], pb[1]);
       const uint32_t gsecond = min3_u32(ps[0], ps[1], max(pb[0], pb[1]));
-      const float vb = bitsf(gbest & 0xffffff00u), vs = bitsf(gsecond & 0xffffff00u);
-      // clear winner: the runner-up more than delta behind (keys are
-      // truncated by less than 2^-15 relative); distances positive and finite
-      const bool clear = (vs - vb * (1.0f + 0x1p-14f) > delta_s) && vb > 0.0f && vb < 3.0e38f &&
+      // tag bits: kg (5:4), t (3:0) -> centroids 16t + 4kg .. + 3
+      const int quad = (int)(((gbest & 0xfu) << 4) | ((gbest >> 2) & 0xcu));
+      // their distances again, one by one: the products' terms in dot products
+      float dq[4];
+      {
+        uint32_t h[4], l[4];
+        transpose_kgroups(yh, h);
+        transpose_kgroups(yl, l);
+        const uint32_t at = ((uint32_t)b * kVmNc + (uint32_t)quad) * 16;
+        const LdsU32x4* const ch = (LdsU32x4*)(lds3 + L.ch() + at);
+        const LdsU32x4* const cl = (LdsU32x4*)(lds3 + L.cl() + at);
+        typedef const __attribute__((address_space(3))) uint32_t LdsU32;
+        const LdsU32* const cq =
+            (LdsU32*)(lds3 + L.cq() + ((uint32_t)(b >> 2) * kVmNc + (uint32_t)quad) * 16 + (uint32_t)(b & 3) * 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const u32x4 hj = ch[j], lj = cl[j];
+          float a = dot2(cq[4 * j], 0x74007400u, init);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) a = dot2(hj[e], h[e], a);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) a = dot2(hj[e], l[e], a);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) a = dot2(lj[e], h[e], a);
+          dq[j] = a;
+        }
+      }
+      const float lo0 = fminf(dq[0], dq[1]), lo1 = fminf(dq[2], dq[3]);
+      const float m1 = fminf(lo0, lo1);
+      const float m2 = fminf(fminf(fmaxf(lo0, lo1), fmaxf(dq[0], dq[1])), fmaxf(dq[2], dq[3]));
+      const float vb = bitsf(gbest & 0xffffffc0u), vs = bitsf(gsecond & 0xffffffc0u);
+      // clear winner: the runner-up among the four and the nearest of any
+      // other four (whose keys are cut downwards) more than delta behind;
+      // distances positive and finite
+      const bool clear = (fminf(m2, vs) - m1 > delta_s) && vb > 0.0f && vb < 3.0e38f &&
                          delta_s < 3.0e38f;
-      // tag bits: kg (7:6), t (5:2), i (1:0) -> centroid 16t + 4kg + i
-      const uint32_t tag = gbest & 0xffu;
-      int idx = (int)(((tag & 0x3cu) << 2) | ((tag >> 4) & 0xcu) | (tag & 3u));
+      int idx = quad + (lo0 <= lo1 ? (dq[0] <= dq[1] ? 0 : 1) : (dq[2] <= dq[3] ? 2 : 3));
       // exact recount of the unclear tokens, one at a time by the whole wave
       uint64_t todo = __ballot(!clear && valid);
       while (todo) {

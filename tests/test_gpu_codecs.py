@@ -565,3 +565,25 @@ def test_blockvq_divided_rows_match_the_whole(dev, nb):
         at += n
     _native.encode_blockvq(k[at:], E, C, ties=t_cut)
     assert t_cut.value() == t_all.value()
+
+
+@pytest.mark.parametrize("eps", [0.0, 1e-7, 3e-6, 1e-4, 1e-2])
+def test_blockvq_near_centroids_in_and_across_quads(dev, eps):
+    """Four centroids close together, beside each other (one product's quad of
+    rows) or apart: the matrix-core encoder's indices and tie count are those
+    of the scan (rows whose stride is no multiple of 16 bytes take it)."""
+    g = torch.Generator().manual_seed(77)
+    base = torch.randn(4, 64, 8, generator=g)
+    near = base[:, :, None, :] + eps * torch.randn(4, 64, 4, 8, generator=g)
+    C = torch.stack([near[0].reshape(256, 8), near[1].transpose(0, 1).reshape(256, 8),
+                     near[2].reshape(256, 8)[torch.randperm(256, generator=g)], near[3].reshape(256, 8)]).to(dev)
+    E = torch.eye(8, device=dev).repeat(4, 1, 1).contiguous()
+    pick = torch.randint(0, 64, (4, 777), generator=g)
+    k = torch.cat([base[b][pick[b]] for b in range(4)], dim=-1)
+    k = (k + torch.randn(777, 32, generator=g) * torch.tensor([1e-3, 0.1, 1.0]).repeat(259)[:, None]).to(dev)
+    strided = torch.empty(777, 33, device=dev)[:, :32].copy_(k)
+    t_mfma, t_scan = _native.TieCounter(dev), _native.TieCounter(dev)
+    got = _native.encode_blockvq(k, E, C, ties=t_mfma)
+    ref = _native.encode_blockvq(strided, E, C, ties=t_scan)
+    assert torch.equal(got, ref)
+    assert t_mfma.value() == t_scan.value()
