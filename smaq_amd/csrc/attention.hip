@@ -492,7 +492,7 @@ static Plan make_plan(const smaq_attn_params* p, bool allow_rows) {
   pl.prefill = (p->impl == 0 || p->impl == 3) && !pl.mfma && prefill_mfma_supported(*p);
   // The row kernel merges the recent window's partials, so that phase has to
   // be in the same call.  It wins wherever it is supported: 37x at 16 x 32768
-  // tokens, 43x at 64 paged sequences (attention_rows.h), 2.9x for the whole
+  // tokens, 43x at 64 paged sequences (attention_rows.h), 12x for the whole
   // call at 5 query tokens over 4001, and down to 16 tokens (28/4 heads, plan
   // alone: 33 against 46 us of scalar keys, 23 against 37 of block-VQ).
   const int phase_mask = p->phases ? p->phases : 15;

@@ -41,7 +41,7 @@
 // token l of the set in lane l, which forms the nearest quad's four distances
 // again from the LDS codebook (the same terms, v_dot2_f32_f16: at most 2^-23 S
 // for each of 13 steps, 1.6e-6) for the clear test, the index, the store and
-// the exact recount.  VALU bound (81 % of the cycles of 16 waves per CU); value
+// the exact recount.  VALU bound (77 % of the busy cycles), with the LDS busy half of them; value
 // and index of every single distance took 30 % more VALU instructions:
 // 4,194,304 rows of 16 blocks, their value pack included, 2253 -> 2116 us.
 #include "encode_internal.h"

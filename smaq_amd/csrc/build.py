@@ -25,7 +25,7 @@ OBJ_DIR = PKG / "_build"
 ARCH = os.environ.get("SMAQ_OFFLOAD_ARCH", "gfx950")
 
 # -ffp-contract=off: the encoders reproduce torch-CPU rounding, so no implicit
-# multiply-add fusion.  Packed FP32 VALU forms are disabled on this pool.
+# multiply-add fusion.  Packed FP32 VALU forms stay disabled (some have given wrong results).
 HIPCC_FLAGS = [
     f"--offload-arch={ARCH}",
     "-O3",
