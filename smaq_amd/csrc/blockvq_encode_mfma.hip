@@ -465,12 +465,13 @@ __global__ __launch_bounds__(kVmThreads) void encode_blockvq_mfma_kernel(
         const auto pb = __builtin_amdgcn_permlane32_swap(best[h], best[h + 2], false, false);
         const auto ps = __builtin_amdgcn_permlane32_swap(second[h], second[h + 2], false, false);
         mb[h] = min(pb[0], pb[1]);
-        ms[h] = min3_u32(ps[0], ps[1], max(pb[0], pb[1]));
+        // (plain code: the compiler places the waits before the next swap)
+        ms[h] = min(min(ps[0], ps[1]), max(pb[0], pb[1]));
       }
       const auto pb = __builtin_amdgcn_permlane16_swap(mb[0], mb[1], false, false);
       const auto ps = __builtin_amdgcn_permlane16_swap(ms[0], ms[1], false, false);
       const uint32_t gbest = min(pb[0], pb[1]);
-      const uint32_t gsecond = min3_u32(ps[0], ps[1], max(pb[0], pb[1]));
+      const uint32_t gsecond = min(min(ps[0], ps[1]), max(pb[0], pb[1]));
       // tag bits: kg (5:4), t (3:0) -> centroids 16t + 4kg .. + 3
       const int quad = (int)(((gbest & 0xfu) << 4) | ((gbest >> 2) & 0xcu));
       // their distances again, one by one: the products' terms in dot products
