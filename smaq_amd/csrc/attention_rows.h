@@ -493,8 +493,12 @@ __global__ __launch_bounds__(RowsKey<KEY>::kWaves * 64)
       qmax = fmaxf(qmax, __shfl_xor(qmax, 16, 64));
       qmax = fmaxf(qmax, __shfl_xor(qmax, 32, 64));
       const int e_q = exponent_of(qmax) - 13;
-      const float qs = ldexpf(1.0f, -e_q);
-      rfac = p.scale * kLog2e * ldexpf(1.0f, e_q + e_k);
+      // The scores are masked (-inf) and their largest found ahead of `rfac`,
+      // which has to be positive: the sign of a negative scale goes into the
+      // query, and so does a scale of zero or NaN.
+      const bool positive = p.scale > 0.0f, negative = p.scale < 0.0f;
+      const float qs = ldexpf(positive ? 1.0f : negative ? -1.0f : p.scale, -e_q);
+      rfac = fmaxf(ldexpf((positive || negative ? fabsf(p.scale) : 1.0f) * kLog2e, e_q + e_k), 0x1p-126f);
       // the hi (first half) or lo part, met with the keys' hi and lo parts
       uint32_t xw[16];
 #pragma unroll

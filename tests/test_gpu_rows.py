@@ -157,3 +157,21 @@ def test_unrotated_query_is_widened_by_the_library(dev, T, rn, impl, dtype):
     assert torch.equal(plan.run_into(strided, torch.empty_like(plan.out)), ref)
     plan.q_exact.fill_(float("nan"))
     assert torch.equal(plan.run_into(q, torch.empty_like(plan.out)), ref)
+
+
+@pytest.mark.parametrize("scale", [0.0, -0.05, 1e-42])
+@pytest.mark.parametrize("codec,size,vbits,g,T,dtype", [FORMS[0], FORMS[3], FORMS[4], FORMS[6]])
+def test_rows_any_scale(dev, codec, size, vbits, g, T, dtype, scale):
+    """A score scale that is zero, negative or below fp32's normal range:
+    tokens past the length or the causal limit stay masked."""
+    strat = _strategy(dev, codec, size)
+    for n, rn in ((77, 0), (300, 9)):
+        st = S.CompressedKVStore(128, 2, value_bits=vbits, device=dev, key_strategy=strat)
+        k = sample_keys(n * 2, seed=n).view(n, 2, 128).to(dtype).to(dev)
+        v = torch.randn(n, 2, 128, generator=torch.Generator().manual_seed(n)).to(dtype).to(dev)
+        st.append_chunk(k, v)
+        q = sample_keys(T * 2 * g, seed=n + 1).view(T, 2 * g, 128).to(dev)
+        kr = sample_keys(max(rn, 1) * 2, seed=n + 2).view(-1, 2, 128).to(dtype).to(dev) if rn else None
+        pos = torch.arange(n + rn - T, n + rn, device=dev) if T > 1 else None
+        got, ref = (S.compute_hybrid_attention(q, st, kr, kr, 2 * g, scale=scale, query_positions=pos, impl=i) for i in (0, 1))
+        _close(got, ref, (v,) if kr is None else (v, kr), f"{codec}{size} g{g} T{T} n{n} r{rn} scale {scale}")
