@@ -24,8 +24,9 @@
 //   soft a lane keeps the four tokens of its column's half (columns 0-7 the
 //        first, 8-15 the second): the scores need one rotation by 8 lanes,
 //        and no LDS.  Base 2, reference raised lazily (attention_mfma.hip),
-//        lowered by the exponent of the largest value scale so that
-//        weight * scale stays inside f16.
+//        lowered by the exponent of the largest weight * scale so that those
+//        products stay inside f16, whatever the scales of tokens of little
+//        weight; value groups far apart get a power of two each.
 //   PV   v_mfma_f32_16x16x32_f16, O^T = V^T P^T per value group: B is
 //        weight * scale split f16 hi (columns 0-7) / lo (8-15), ~22 bits,
 //        which the softmax lanes hold in place (the tokens of the K slots are
@@ -67,6 +68,19 @@ struct RowsKey {
   static constexpr int kTable = kVq ? 128 * 256 * 4 : 256 * 8;
   static constexpr int kWaves = kVq ? 8 : 4;                  // per workgroup
 };
+
+// The f16 pairs of weight * scale: a row's largest product so far is brought
+// to [2^kPairExp, 2^(kPairExp + 1)) and may come to 2^kPairTop (and 0.09 of an
+// octave, the error of a log2 taken from a number's bits; f16 ends at 2^16)
+// before the exponent follows.  A pair holds 22 bits of a product and multiples
+// of 2^-24, so a value group's sum keeps 28 bits or more below its largest
+// product (with kPairApart); a higher kPairExp costs the weights' exponents bits.
+// (One exponent that followed the largest scale alone lost 2e-3 of the other
+// groups beside a channel 1e6 times theirs.  Following products, group by group:
+// 64 paged sequences of heavy-tailed keys 62.7 -> 64.0 us, other calls the same.)
+constexpr int kPairExp = 6;
+constexpr float kPairTop = 15.5f;
+constexpr int kPairApart = 2;
 
 // buffer-load policy sc1: agent-coherent, as load_agent
 constexpr int kAgentPolicy = 16;
@@ -125,6 +139,18 @@ __device__ __forceinline__ void rows_split2(float x0, float x1, float one, uint3
   const f32x2 r = {__builtin_fmaf(one, x0, -(float)h[0]), __builtin_fmaf(one, x1, -(float)h[1])};
   hi = __builtin_bit_cast(uint32_t, h);
   lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, rf16x2));
+}
+
+// the largest of a query row's 8 lanes (n, n ^ 8 in each 16-lane row)
+__device__ __forceinline__ float rows_max8(float x) {
+  auto number = [](uint32_t bits) -> float { return __builtin_bit_cast(float, bits); };
+  x = fmaxf(x, dpp_row_ror<0x128>(x));
+  uint32_t b = __builtin_bit_cast(uint32_t, x);
+  const auto p = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  x = fmaxf(number(p[0]), number(p[1]));
+  b = __builtin_bit_cast(uint32_t, x);
+  const auto q = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+  return fmaxf(number(q[0]), number(q[1]));
 }
 
 template <int CTRL, int BANKS>
@@ -614,8 +640,14 @@ __global__ __launch_bounds__(RowsKey<KEY>::kWaves * 64)
     // the sums this lane's share)
     float m_run = -__builtin_inff(), m_thr = -__builtin_inff();
     float mref = -__builtin_inff(), mexp = 0.0f;   // reference, and as the exponent takes it
-    int e_s = -40;
-    float s_thr = 0.0f;                            // scales above it raise e_s
+    // Products weight * scale as f16 pairs: e_fold is the exponent, relative to
+    // m_run, of the row's largest (the weights carry 2^(kPairExp - e_fold)),
+    // eg that of each value group's.  `apart`: some row's groups are more than
+    // 2^kPairApart apart, and a group's products move by its own power of two.
+    int e_fold = 0, eg[4] = {-127, -127, -127, -127};
+    bool apart = false;
+    float p_thr = 0.0f;                            // log2 products (plus 127) that need a look: any, with `apart`
+    auto shift_of = [&](int gg) -> int { return min(max(e_fold - eg[gg], -100), 100); };
     float l_run = 0.0f;
     float zacc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     f32x4 acc[8];                                  // [value group][code field]
@@ -682,37 +714,87 @@ __global__ __launch_bounds__(RowsKey<KEY>::kWaves * 64)
 #pragma unroll
         for (int v = 0; v < 4; ++v) xs[v] = tok0 + v > lim ? -__builtin_inff() : xs[v];
       }
-      float sv[16];
-      float smax = 0.0f;
+      // scales, and what a unit weight adds to the fp32 sums
+      float sv[16], zz[16];
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         sv[i] = packed_get<TV>(sw, i);
-        smax = fmaxf(smax, sv[i]);
+        zz[i] = fmaf(kMid, sv[i], packed_get<TV>(zw, i));
+        asm volatile("" : "+v"(zz[i]));  // (here, so that `sv` may be scaled in place)
       }
       const float tmax = fmaxf(fmaxf(xs[0], xs[1]), fmaxf(xs[2], xs[3])) * rfac;
-      if (__any(tmax > m_thr || smax > s_thr)) {
-        float mt = fmaxf(tmax, dpp_row_ror<0x128>(tmax));
-        mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
-        mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-        float sm = smax;
+      // whether a score or a product is past what the references hold for
+      auto grown = [&](float thr) -> bool {
+        float smax = 0.0f;
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) sm = fmaxf(sm, __shfl_xor(sm, o, 64));
-        // the exponent of the largest scale so far, kept where the weights
-        // stay far inside fp32's range
-        const int e_new = min(max((int)((__builtin_bit_cast(uint32_t, sm) >> 23) & 0xffu) - 127, e_s), 100);
-        m_run = fmaxf(m_run, mt);
-        const float r_new = m_run == -__builtin_inff() ? m_run : m_run + (float)(e_new - 6);
-        const float alpha = mref == -__builtin_inff() ? 0.0f : fast_exp2(mref - r_new);
+        for (int i = 0; i < 16; ++i) smax = fmaxf(smax, fabsf(sv[i]));
+        // (a number's bits * 2^-23 - 127 is its log2, less at most 0.09)
+        return __any((tmax > m_thr) | (fmaf((float)__builtin_bit_cast(uint32_t, smax), 0x1p-23f, tmax) > thr));
+      };
+      if (__builtin_expect(grown(p_thr), 0)) {
+        bool grow = true;
+        if (apart) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) acc[i] *= alpha;
+          for (int i = 0; i < 16; ++i) sv[i] = __builtin_amdgcn_ldexpf(sv[i], shift_of(i & 3));
+          grow = grown(mexp + (127.0f + kPairTop));
+        }
+        if (grow) {
+          const bool was = apart;
+          int old[4] = {0, 0, 0, 0};  // the groups' powers of two so far
+          if (was) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) zacc[i] *= alpha;
-        l_run *= alpha;
-        mref = r_new;
-        mexp = r_new == -__builtin_inff() ? 0.0f : r_new;
-        m_thr = m_run + 8.0f;
-        e_s = e_new;
-        s_thr = ldexpf(1.0f, e_new + 1);
+            for (int i = 0; i < 16; ++i) sv[i] = packed_get<TV>(sw, i);
+#pragma unroll
+            for (int gg = 0; gg < 4; ++gg) old[gg] = shift_of(gg);
+          }
+          // the row's largest score, and log2 of each group's largest product
+          // (as above) beside it
+          const float base = tmax == -__builtin_inff() ? 0.0f : tmax;
+          float pg[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const float w = fast_exp2(fmaf(xs[v], rfac, -base));
+#pragma unroll
+            for (int gg = 0; gg < 4; ++gg) pg[gg] = fmaxf(pg[gg], fabsf(w * sv[4 * v + gg]));
+          }
+          const float mt = rows_max8(tmax), m_new = fmaxf(m_run, mt);
+          const int drop = m_new > m_run ? (int)fminf(m_new - m_run, 512.0f) : 0;
+#pragma unroll
+          for (int gg = 0; gg < 4; ++gg) {
+            const float lg = rows_max8(fmaf((float)__builtin_bit_cast(uint32_t, pg[gg]), 0x1p-23f, tmax - 127.0f));
+            eg[gg] = max(eg[gg] - drop, (int)floorf(fmaxf(lg - m_new, -127.0f)));
+          }
+          const int e_max = max(max(eg[0], eg[1]), max(eg[2], eg[3]));
+          const int e_min = min(min(eg[0], eg[1]), min(eg[2], eg[3]));
+          // (clamped where the weights stay far inside fp32's range)
+          e_fold = min(max(e_max, -40), 60);
+          apart = __any((e_fold - e_min > kPairApart || e_fold < e_max) && m_new > -__builtin_inff());
+          m_run = m_new;
+          const float r_new = m_run == -__builtin_inff() ? m_run : m_run + (float)(e_fold - kPairExp);
+          const float by = mref == -__builtin_inff() ? mref : mref - r_new;
+          const float alpha = fast_exp2(by);
+          l_run *= alpha;
+#pragma unroll
+          for (int gg = 0; gg < 4; ++gg) zacc[gg] *= alpha;
+          if (was || apart) {
+#pragma unroll
+            for (int gg = 0; gg < 4; ++gg) {
+              const int to = apart ? shift_of(gg) : 0;
+              const float beta = fast_exp2(by + (float)(to - old[gg]));
+              acc[2 * gg] *= beta;
+              acc[2 * gg + 1] *= beta;
+#pragma unroll
+              for (int v = 0; v < 4; ++v) sv[4 * v + gg] = __builtin_amdgcn_ldexpf(sv[4 * v + gg], to);
+            }
+          } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) acc[i] *= alpha;
+          }
+          mref = r_new;
+          mexp = r_new == -__builtin_inff() ? 0.0f : r_new;
+          m_thr = m_run + 10.0f;
+          p_thr = apart ? -__builtin_inff() : mexp + (127.0f + kPairTop);
+        }
       }
       float pw[4];
 #pragma unroll
@@ -720,8 +802,7 @@ __global__ __launch_bounds__(RowsKey<KEY>::kWaves * 64)
         pw[v] = fast_exp2(fmaf(xs[v], rfac, -mexp));
         l_run += pw[v];
 #pragma unroll
-        for (int gg = 0; gg < 4; ++gg)
-          zacc[gg] = fmaf(pw[v], fmaf(kMid, sv[4 * v + gg], packed_get<TV>(zw, 4 * v + gg)), zacc[gg]);
+        for (int gg = 0; gg < 4; ++gg) zacc[gg] = fmaf(pw[v], zz[4 * v + gg], zacc[gg]);
       }
       // -- O^T, kGroups value groups per pass
 #pragma unroll
@@ -822,13 +903,14 @@ __global__ __launch_bounds__(RowsKey<KEY>::kWaves * 64)
 #pragma unroll
       for (int gi = 0; gi < 2; ++gi) {
         const int gg = 2 * half + gi;
+        const float unit = ldexpf(1024.0f, apart ? -shift_of(gg) : 0);
 #pragma unroll
         for (int f = 0; f < 2; ++f) {
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
             // value row m = 4kg + v: dim 2m + f of the group
             const float a = acc[2 * gg + f][v];
-            const float o = fmaf(a + dpp_row_ror<0x128>(a), 1024.0f, zacc[gg]);
+            const float o = fmaf(a + dpp_row_ror<0x128>(a), unit, zacc[gg]);
             if (first) red_o[wu][q8][32 * gi + 2 * (4 * kg + v) + f] = o;
           }
         }

@@ -175,3 +175,47 @@ def test_rows_any_scale(dev, codec, size, vbits, g, T, dtype, scale):
         pos = torch.arange(n + rn - T, n + rn, device=dev) if T > 1 else None
         got, ref = (S.compute_hybrid_attention(q, st, kr, kr, 2 * g, scale=scale, query_positions=pos, impl=i) for i in (0, 1))
         _close(got, ref, (v,) if kr is None else (v, kr), f"{codec}{size} g{g} T{T} n{n} r{rn} scale {scale}")
+
+
+@pytest.mark.parametrize("how", ["channel 1e4", "channel 1e6", "channel 1e9", "one value 1e9", "infinite scale",
+                                 "token of little weight 1e6", "zero up to a late token"])
+@pytest.mark.parametrize("codec,size,vbits,g,dtype", [("vq", 8, 2, 8, torch.bfloat16), ("scalar", 3, 4, 7, torch.float32)])
+def test_rows_value_groups_far_apart(dev, codec, size, vbits, g, dtype, how):
+    """Each group of 32 value dims is as exact as when it stands alone: one
+    group's scales far above the others', at every token, at one, infinite, at
+    a token of next to no weight, or zero up to a late token.  Tolerance: the
+    file's, of the largest value of the group itself (the light token's left
+    out)."""
+    strat = _strategy(dev, codec, size)
+    n, gen = 1500, torch.Generator().manual_seed(8)
+    k = sample_keys(n * 2, seed=5).view(n, 2, 128).to(dtype).to(dev)
+    v = torch.randn(n, 2, 128, generator=gen)
+    q = 60 * sample_keys(2 * g, seed=6).view(1, 2 * g, 128).to(dev)   # (logits up to 30)
+    live = torch.ones(n, 2, dtype=torch.bool)
+    if how.startswith("channel"):
+        v[:, :, 7] *= float(how.split()[1])
+    elif how == "one value 1e9":
+        v[700, 1, 40] = 1e9
+    elif how == "token of little weight 1e6":
+        khat = strat.dequantize(strat.quantize(k)).float().cpu()
+        logits = torch.einsum("nhd,hgd->nhg", khat, q.cpu().view(2, g, 128)) * 128 ** -0.5
+        light = torch.softmax(logits, 0).amax(2).argmin(0)
+        for h in range(2):
+            v[light[h], h] *= 1e6
+            live[light[h], h] = False
+    elif how == "zero up to a late token":
+        v[:1300, :, 64:96] = 0.0
+    v = v.to(dtype).to(dev)
+    kv = QuantizedKVBatch.encode(strat, [k], [v], value_bits=vbits)
+    if how == "infinite scale":
+        kv.v_scales[1, 700, 2] = float("inf")
+    got, ref = kv.attention(q), kv.attention(q, impl=1)
+    top = (v.float() * live.to(dev).unsqueeze(-1)).view(n, 2, 4, 32).abs().amax((0, 3))   # [Hkv, group]
+    err = (got - ref).view(2, g, 4, 32).abs().amax((1, 3))
+    for h in range(2):
+        for i in range(4):
+            if how == "infinite scale" and (h, i) == (1, 2):
+                assert not got.view(2, g, 4, 32)[h, :, i].isfinite().any()
+                continue
+            print(f"\n[{codec}{size} {how} head {h} group {i}] max|err| {float(err[h, i]):.2e} of {float(top[h, i]):.2e}")
+            assert float(err[h, i]) <= 2e-5 * float(top[h, i])
