@@ -20,7 +20,7 @@
 //        A key code becomes its f16 hi/lo pair by one LDS read of a table of
 //        all codes (scalar keys: 256 code bytes; block-VQ: every codeword of
 //        every block, 128 KB, one workgroup of 8 waves per CU), both halves
-//        scaled by a power of two that keeps the lo part normal.
+//        scaled by a power of two per block that keeps the lo part normal.
 //   soft a lane keeps the four tokens of its column's half (columns 0-7 the
 //        first, 8-15 the second): the scores need one rotation by 8 lanes,
 //        and no LDS.  Base 2, reference raised lazily (attention_mfma.hip),
@@ -325,6 +325,7 @@ __global__ __launch_bounds__(RowsKey<KEY>::kWaves * 64)
   __shared__ __attribute__((aligned(16))) uint8_t vsp[NW][kRowsVBytes * kRowsPitch];
   __shared__ float red_m[NW][kRowsQ], red_l[NW][kRowsQ];
   __shared__ int flag;
+  __shared__ int blk_e[K::kVq ? 128 / KEY : 1];  // the blocks' powers of two
   // per-wave outputs of 64 dims, laid over the value tiles between units
   float (*const red_o)[kRowsQ][64] = (float (*)[kRowsQ][64])&vsp[0][0];
   static_assert(sizeof(vsp[0]) >= sizeof(float) * kRowsQ * 64, "red_o");
@@ -388,18 +389,25 @@ __global__ __launch_bounds__(RowsKey<KEY>::kWaves * 64)
   b = __builtin_amdgcn_readfirstlane(b);
   x_seq = (uint32_t)__builtin_amdgcn_readfirstlane(x_seq);
 
-  // ---- key table, scaled by 2^-e_k so that the largest entry lies in
-  // [2^13, 2^14): the lo parts of entries down to 2^-17 of it are normal f16
-  int e_k;
+  // ---- key table, each block (scalar keys: all of it) scaled by a power of two
+  // that brings its largest entry to [2^13, 2^14): the lo parts of entries down
+  // to 2^-17 of it are normal f16.  A block's own power goes into the query's
+  // dims, so blocks of any size count alike.
+  auto finite = [](float x) -> float { return fabsf(x) < __builtin_inff() ? fabsf(x) : 0.0f; };
+  auto exponent = [](float x) -> int { return max(exponent_of(x) - 13, -126); };
+  int e_k = 0;
   if constexpr (K::kVq) {
-    constexpr int kPer = 128 * 256 / KEY / kThreads;  // codewords per thread
+    constexpr int kTpb = kThreads * KEY / 128;  // threads of a block
+    constexpr int kPer = 256 / kTpb;            // codewords per thread
     const int nc = p.vq_centroids;
+    const int blk = tid / kTpb, sub = tid % kTpb;
+    // (rotated by block, so that a wave's writes cover all LDS banks)
+    auto code = [&](int i) -> int { return sub + kTpb * ((i + blk) % kPer); };
     float c[kPer][KEY];
     float cmax = 0.0f;
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
-      const int e = tid + i * kThreads, blk = e >> 8, ci = min(e & 255, nc - 1);
-      const float* src = p.key_lut + ((int64_t)blk * nc + ci) * KEY;
+      const float* src = p.key_lut + ((int64_t)blk * nc + min(code(i), nc - 1)) * KEY;
       if constexpr (KEY == 2) {
         const float2 v = *(const float2*)src;
         c[i][0] = v.x; c[i][1] = v.y;
@@ -411,19 +419,16 @@ __global__ __launch_bounds__(RowsKey<KEY>::kWaves * 64)
         }
       }
 #pragma unroll
-      for (int d = 0; d < KEY; ++d) cmax = fmaxf(cmax, fabsf(c[i][d]));
+      for (int d = 0; d < KEY; ++d) cmax = fmaxf(cmax, finite(c[i][d]));
     }
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) cmax = fmaxf(cmax, __shfl_xor(cmax, o, 64));
-    if (lane == 0) red_m[wu][0] = cmax;
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < NW; ++w) cmax = fmaxf(cmax, red_m[w][0]);
-    e_k = exponent_of(cmax) - 13;
-    const float ks = ldexpf(1.0f, -e_k);
+    for (int o = 1; o < kTpb; o <<= 1) cmax = fmaxf(cmax, __shfl_xor(cmax, o, 64));
+    const int e_b = exponent(cmax);
+    if (sub == 0) blk_e[blk] = e_b;
+    const float ks = ldexpf(1.0f, -e_b);
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
-      const int e = tid + i * kThreads;
+      const int e = blk * 256 + code(i);
       uint32_t hi[KEY / 2], lo[KEY / 2];
 #pragma unroll
       for (int d = 0; d < KEY; d += 2) rows_split2(c[i][d] * ks, c[i][d + 1] * ks, one, hi[d / 2], lo[d / 2]);
@@ -437,8 +442,8 @@ __global__ __launch_bounds__(RowsKey<KEY>::kWaves * 64)
   } else {
     const int nc = 1 << p.key_bits;
     float cmax = 0.0f;
-    for (int i = 0; i < nc; ++i) cmax = fmaxf(cmax, fabsf(p.key_lut[i]));
-    e_k = exponent_of(cmax) - 13;
+    for (int i = 0; i < nc; ++i) cmax = fmaxf(cmax, finite(p.key_lut[i]));
+    e_k = exponent(cmax);
     const float ks = ldexpf(1.0f, -e_k);
     static_assert(K::kVq || kThreads == 256, "one table entry per thread");
     uint32_t hi, lo;
@@ -514,11 +519,12 @@ __global__ __launch_bounds__(RowsKey<KEY>::kWaves * 64)
 #pragma unroll
       for (int i = 0; i < 32; ++i) {
         qv[i] = q8 < nr ? qv[i] : 0.0f;
+        if constexpr (K::kVq) qv[i] = __builtin_amdgcn_ldexpf(qv[i], blk_e[(32 * kg + i) / KEY]);
         qmax = fmaxf(qmax, fabsf(qv[i]));
       }
       qmax = fmaxf(qmax, __shfl_xor(qmax, 16, 64));
       qmax = fmaxf(qmax, __shfl_xor(qmax, 32, 64));
-      const int e_q = exponent_of(qmax) - 13;
+      const int e_q = exponent(qmax);
       // The scores are masked (-inf) and their largest found ahead of `rfac`,
       // which has to be positive: the sign of a negative scale goes into the
       // query, and so does a scale of zero or NaN.

@@ -219,3 +219,32 @@ def test_rows_value_groups_far_apart(dev, codec, size, vbits, g, dtype, how):
                 continue
             print(f"\n[{codec}{size} {how} head {h} group {i}] max|err| {float(err[h, i]):.2e} of {float(top[h, i]):.2e}")
             assert float(err[h, i]) <= 2e-5 * float(top[h, i])
+
+
+@pytest.mark.parametrize("what", ["queries 2^-118", "queries 2^-130", "codebook 2^-118", "one block 2^40", "one block 2^-40"])
+@pytest.mark.parametrize("size", [2, 4, 8])
+def test_rows_query_and_codebook_range(dev, size, what):
+    """Queries and codebooks at the edge of fp32's range (the score scale makes
+    up for it), and a block whose codewords are far larger or smaller than the
+    others' with its query dims the inverse: every block counts alike."""
+    strat = _strategy(dev, "vq", size)
+    n, g, nb = 333, 4, 128 // size
+    k = sample_keys(n * 2, seed=5).view(n, 2, 128)
+    v = torch.randn(n, 2, 128, generator=torch.Generator().manual_seed(4))
+    kv = QuantizedKVBatch.encode(strat, [k.to(dev)], [v.to(dev)])
+    q = sample_keys(2 * g, seed=6).view(1, 2 * g, 128).to(dev)
+    scale, power = 128 ** -0.5, what.split("2^")[1]
+    f = 2.0 ** int(power)
+    state = strat.quantizer.state_dict()
+    C = state["decoded_centroids"].clone()
+    if what.startswith("queries"):
+        q, scale = q * f, scale * 2.0 ** min(-int(power), 126)
+    elif what.startswith("codebook"):
+        C, scale = C * f, scale / f
+    else:
+        C[nb // 2] *= f
+        q.view(1, 2 * g, nb, size)[:, :, nb // 2] /= f
+    strat.quantizer.load_state_dict({**state, "decoded_centroids": C})
+    got, ref = (kv.attention(q, scale=scale, impl=i) for i in (0, 1))
+    assert float((ref - ref.mean(1, keepdim=True)).abs().max()) > 1e-3
+    _close(got, ref, (v,), f"vq{size} {what}")
