@@ -313,7 +313,11 @@ typedef struct smaq_attn_params {
      phases 8 and 1 run in one call); with 16 added,
      phase 1 reuses the schedule an earlier call on this workspace built for
      the same lengths, so the decode kernel can be timed alone (with any
-     other workspace contents the output is undefined).  32 added to the
+     other workspace contents the output is undefined).  The row kernel (see
+     impl) writes the output itself too: without a recent part in phase 1, with
+     one only in a call that launches phases 1, 2 and 4 together (or all); a
+     call with some of them runs the generic kernels, whose partials the later
+     phases read.  After a complete call phase 4 has nothing to read.  32 added to the
      phases wanted: q_raw is first written to q_exact as fp32 (by the recent
      window's kernel when that one runs first, else by one launch), so a
      caller with rot_mt NULL and q_hist = q_exact hands in the query as it

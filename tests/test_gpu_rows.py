@@ -248,3 +248,28 @@ def test_rows_query_and_codebook_range(dev, size, what):
     got, ref = (kv.attention(q, scale=scale, impl=i) for i in (0, 1))
     assert float((ref - ref.mean(1, keepdim=True)).abs().max()) > 1e-3
     _close(got, ref, (v,), f"vq{size} {what}")
+
+
+@pytest.mark.parametrize("codec,size,vbits,g,T,dtype", [FORMS[0], FORMS[4], FORMS[6]])
+@pytest.mark.parametrize("rn", [0, 70])
+def test_rows_shapes_in_separate_phases(dev, codec, size, vbits, g, T, dtype, rn):
+    """Phases launched apart, whichever are joined, give the generic kernels'
+    result."""
+    strat = _strategy(dev, codec, size)
+    n = 400
+    k = sample_keys(2 * n * 2, seed=1).view(2, n, 2, 128).to(dtype).to(dev)
+    v = torch.randn(2, n, 2, 128, generator=torch.Generator().manual_seed(2)).to(dtype).to(dev)
+    kv = QuantizedKVBatch.encode(strat, k, v, value_bits=vbits)
+    q = sample_keys(2 * T * 2 * g, seed=3).view(2, T, 2 * g, 128).to(dev)
+    rk = sample_keys(2 * rn * 2, seed=4).view(2, rn, 2, 128).to(dtype).to(dev) if rn else None
+    rl = torch.tensor([rn, rn // 2], device=dev) if rn else None
+    ref = kv.plan(q, None, rk, rk, rl, impl=1).run(q)
+    plan = kv.plan(q, None, rk, rk, rl)
+    vals = (v,) if rk is None else (v, rk)
+    _close(plan.run(q), ref, vals, "one call")
+    for masks in ((8, 1, 2, 4), (8 | 1 | 2, 4), (8, 1, 2 | 4), (8 | 2, 1 | 4), (8, 1 | 2 | 4)):
+        plan.load_query(q)
+        plan.out.fill_(float("nan"))
+        for m in masks:
+            plan.launch(m)
+        _close(plan.out, ref, vals, f"{codec}{size} T{T} r{rn} phases {masks}")
