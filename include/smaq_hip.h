@@ -367,7 +367,10 @@ typedef struct smaq_attn_params {
   long long hist_rows;
 } smaq_attn_params;
 
-/* Bytes of workspace smaq_attn_hybrid needs for these parameters. */
+/* Bytes of workspace with which smaq_attn_hybrid has its choice of kernels for
+ * these parameters.  Sized with arrivals NULL it is what the other kernels
+ * need: with that much, and less than the row kernel needs, a call that would
+ * take the row kernel runs the generic ones. */
 long long smaq_attn_workspace_bytes(const smaq_attn_params* p);
 int smaq_attn_hybrid(const smaq_attn_params* p, void* stream);
 
@@ -377,9 +380,10 @@ int smaq_attn_hybrid(const smaq_attn_params* p, void* stream);
  * capture, serving loops that forbid hipMalloc).  Same kernels and results as
  * smaq_attn_hybrid; p->workspace and p->workspace_bytes are ignored and the
  * workspace is a built-in device array of SMAQ_NOALLOC_SCRATCH_BYTES per GPU,
- * held until the process ends.  Parameters whose smaq_attn_workspace_bytes
- * exceeds that size are rejected with SMAQ_EINVAL (decode batches fit; the
- * matrix-core prefill's tile images generally do not).  Nothing in the array
+ * held until the process ends.  Parameters whose smaq_attn_workspace_bytes with
+ * arrivals NULL exceeds that size are rejected with SMAQ_EINVAL (decode batches
+ * fit; the matrix-core prefill's tile images generally do not); where only the
+ * row kernel's workspace exceeds it, the generic kernels run.  Nothing in the array
  * needs clearing between calls (every partial a call reads it writes first),
  * but calls that overlap on one GPU -- on two streams, or two threads --
  * share the array and race.  The first call on a device looks up the array's

@@ -16,6 +16,7 @@
 // Score arithmetic follows the reference per segment: scalar history
 // ((q_rot . c[code]) * norm) * scale, block-VQ (q . k_hat) * scale, recent
 // (q . k) * scale, all fp32.
+#include <algorithm>
 #include <math.h>
 
 #include "attention_internal.h"
@@ -583,15 +584,12 @@ static int64_t plan_bytes(const smaq_attn_params* p, const Plan& pl) {
 }
 
 // Whatever the phases of the calls that share the workspace: enough for the
-// generic kernels, and for the row kernel unless that alone would pass the
-// built-in scratch's size.
+// generic kernels and for the row kernel.
 extern "C" long long smaq_attn_workspace_bytes(const smaq_attn_params* p) {
   if (!p || p->n_kv_heads <= 0 || p->n_q_heads % p->n_kv_heads) return -1;
   const int64_t bytes = plan_bytes(p, make_plan(p, false));
   const Plan rows = make_plan(p, true);
-  if (!rows.rows) return bytes;
-  const int64_t more = plan_bytes(p, rows);
-  return more <= bytes || (more > SMAQ_NOALLOC_SCRATCH_BYTES && bytes <= SMAQ_NOALLOC_SCRATCH_BYTES) ? bytes : more;
+  return rows.rows ? std::max(bytes, plan_bytes(p, rows)) : bytes;
 }
 
 template <int KEY, typename TN, typename TV>
@@ -888,8 +886,10 @@ static int scratch_for_stream(hipStream_t st, void** out) {
 
 extern "C" int smaq_attn_hybrid_noalloc(const smaq_attn_params* pp, void* stream) {
   SMAQ_REQUIRE(pp, "smaq_attn_hybrid_noalloc: null params");
-  const long long need = smaq_attn_workspace_bytes(pp);
-  SMAQ_REQUIRE(need >= 0, "smaq_attn_hybrid_noalloc: invalid parameters");
+  SMAQ_REQUIRE(smaq_attn_workspace_bytes(pp) >= 0, "smaq_attn_hybrid_noalloc: invalid parameters");
+  // (the row kernel's partials, a slot of 8 rows for every unit, are the larger:
+  // a call that has no room for them runs the generic kernels)
+  const long long need = plan_bytes(pp, make_plan(pp, false));
   SMAQ_REQUIRE(need <= smaq::kNoAllocScratchBytes,
                "smaq_attn_hybrid_noalloc: these shapes need %lld bytes of workspace, more than the %lld-byte "
                "built-in scratch; use smaq_attn_hybrid with a caller workspace",

@@ -273,3 +273,29 @@ def test_rows_shapes_in_separate_phases(dev, codec, size, vbits, g, T, dtype, rn
         for m in masks:
             plan.launch(m)
         _close(plan.out, ref, vals, f"{codec}{size} T{T} r{rn} phases {masks}")
+
+
+def test_rows_past_the_built_in_scratch(dev):
+    """A batch whose row-kernel workspace passes the allocation-free entry
+    point's scratch: a plan owns its workspace and takes the row kernel; the
+    allocation-free call, whose generic workspace fits, still runs."""
+    import ctypes
+    from smaq_amd import _native
+    strat = _strategy(dev, "vq", 8)
+    B, H, n, g = 700, 16, 40, 1
+    k = sample_keys(n * H, seed=1).view(1, n, H, 128).to(dev) + 0.1 * torch.randn(
+        B, 1, H, 1, generator=torch.Generator().manual_seed(3)).to(dev)
+    kv = QuantizedKVBatch.encode(strat, k, k)
+    q = sample_keys(B * H * g, seed=2).view(B, H * g, 128).to(dev)
+    plan = kv.plan(q)
+    generic = kv.plan(q, impl=1).params.workspace_bytes
+    slots = B * H * 8 * 130 * 4
+    assert generic < _native.NOALLOC_SCRATCH_BYTES < slots
+    assert plan.params.workspace_bytes > slots
+    got, ref = plan.run(q).clone(), kv.attention(q, impl=1).view_as(plan.out)
+    _close(got, ref, (k,), "700 x 16 units")
+    assert not torch.equal(got, ref)       # (the row kernel's sums, not the generic one's)
+    plan.load_query(q)
+    plan.out.fill_(float("nan"))
+    _native.attn_hybrid_noalloc(plan.params, dev)
+    assert torch.equal(plan.out, ref)
