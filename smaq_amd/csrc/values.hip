@@ -218,6 +218,51 @@ static int launch_dequant(const void* data, const void* scales, const void* zero
 constexpr int kAvThreads = 256;
 constexpr int kAvQ = 4;         // query rows per pass over the tokens
 constexpr int kAvMaxD = 512;
+// A workgroup of the exact rows (smaq_cache_attend): kAvXRows of them for kAvXQ
+// query rows, so that a long window or many query rows fill the device (one
+// workgroup a lane for the whole window and every query row: 16 lanes of 8064
+// tokens, window 4096, one row 80 us, 8 rows 508, 64 rows 3985; now 29, 74, 431.
+// A row of a window of 128 as before, 17 us).
+constexpr int kAvXRows = 256;
+constexpr int kAvXQ = 8;
+
+// to[q][d] = sum over r < nr of wq[q][r] rows[r][d], q < nqq <= Q.  A thread sums
+// one dim over a share of the rows (D <= 256: 256 / D shares); the weights are
+// staged by row, so that a row's are one or two LDS reads.
+template <int Q>
+__device__ __forceinline__ void exact_rows(float* lds, const float* wq, int64_t w_qstride, int nqq, const float* rows,
+                                           int nr, int D, float* to) {
+  const int tid = threadIdx.x;
+  float* const wl = lds;                    // [kAvXRows][Q]
+  float* const sum = lds + kAvXRows * Q;    // [Q][shares * D]
+  if (tid < nr)
+#pragma unroll
+    for (int q = 0; q < Q; ++q) wl[tid * Q + q] = q < nqq ? wq[(int64_t)q * w_qstride + tid] : 0.0f;
+  __syncthreads();
+  const int shares = D <= kAvThreads ? kAvThreads / D : 1;
+  for (int i = tid; i < shares * D; i += kAvThreads) {
+    const int d = i % D;
+    float a[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) a[q] = 0.0f;
+#pragma unroll 16
+    for (int r = i / D; r < nr; r += shares) {
+      const float v = rows[(int64_t)r * D + d];
+#pragma unroll
+      for (int q = 0; q < Q; ++q) a[q] = __builtin_fmaf(wl[r * Q + q], v, a[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) sum[q * shares * D + i] = a[q];
+  }
+  __syncthreads();
+  for (int i = tid; i < nqq * D; i += kAvThreads) {
+    const int q = i / D, d = i - q * D;
+    float a = sum[q * shares * D + d];
+    for (int k = 1; k < shares; ++k) a += sum[(q * shares + k) * D + d];
+    to[i] = a;
+  }
+}
+static_assert(kAvXRows == kAvThreads && kAvXRows * kAvXQ + kAvXQ * kAvMaxD <= 4 * kAvQ * kAvMaxD, "LDS of the exact rows");
 
 template <int VPB, typename T>
 __global__ __launch_bounds__(kAvThreads) void apply_values_kernel(
@@ -243,28 +288,17 @@ __global__ __launch_bounds__(kAvThreads) void apply_values_kernel(
   const float* wb = w + (int64_t)b * w_bstride;
   float* pout = part + (int64_t)s * part_split + (int64_t)b * nq * D;
   if (s >= n_splits) {
-    // the split past the packed ones: R exact rows, weights N .. N + R - 1.  A
-    // thread sums one dim over a share of the rows (D <= 256: 256 / D shares)
-    float (*const sum)[kAvMaxD] = red[0];
-    const float* const rows = xv + (int64_t)b * xv_bstride;
-    const int shares = D <= kAvThreads ? kAvThreads / D : 1;
-    for (int q = 0; q < nq; ++q) {
-      const float* const wq = wb + (int64_t)q * w_qstride + N;
-      for (int i = tid; i < shares * D; i += kAvThreads) {
-        const int d = i % D;
-        float a = 0.0f;
-#pragma unroll 16
-        for (int64_t r = i / D; r < R; r += shares) a = __builtin_fmaf(wq[r], rows[r * D + d], a);
-        (&sum[0][0])[i] = a;
-      }
-      __syncthreads();
-      for (int d = tid; d < D; d += kAvThreads) {
-        float a = (&sum[0][0])[d];
-        for (int k = 1; k < shares; ++k) a += (&sum[0][0])[k * D + d];
-        pout[(int64_t)q * D + d] = a;
-      }
-      __syncthreads();
-    }
+    // past the packed splits: splits of the exact rows, one after another for
+    // each tile of query rows
+    const int xs = (int)((R + kAvXRows - 1) / kAvXRows), x = s - n_splits;
+    const int64_t r0 = (int64_t)(x % xs) * kAvXRows;
+    const int q0 = (x / xs) * kAvXQ;
+    const float* const wq = wb + (int64_t)q0 * w_qstride + N + r0;
+    const float* const rows = xv + (int64_t)b * xv_bstride + r0 * D;
+    const int nr = (int)min((int64_t)kAvXRows, R - r0);
+    float* const to = part + (int64_t)(n_splits + x % xs) * part_split + ((int64_t)b * nq + q0) * D;
+    if (nq == 1) exact_rows<1>(&red[0][0][0], wq, w_qstride, 1, rows, nr, D, to);
+    else exact_rows<kAvXQ>(&red[0][0][0], wq, w_qstride, min(kAvXQ, nq - q0), rows, nr, D, to);
     return;
   }
   for (int q0 = 0; q0 < nq; q0 += kAvQ) {
@@ -388,6 +422,8 @@ extern "C" long long smaq_apply_values_workspace_bytes(long long batch, long lon
   return n_splits > 1 ? (long long)(n_splits * batch * nq * D * (int64_t)sizeof(float)) : 0;
 }
 
+static int64_t exact_splits(long long R) { return R > 0 ? (R + kAvXRows - 1) / kAvXRows : 0; }
+
 static int apply_values(const float* w, long long w_bstride, long long w_qstride, long long batch, long long nq,
                         long long N, int D, const void* data, long long d_bstride, int bits, int group,
                         const void* scales, const void* zeros, long long s_bstride, int sdtype, long long R,
@@ -404,7 +440,7 @@ extern "C" int smaq_apply_values(const float* w, long long w_bstride, long long 
 
 extern "C" long long smaq_cache_attend_workspace_bytes(long long batch, long long nq, long long N, long long R, int D) {
   if (batch <= 0 || nq <= 0 || D <= 0) return 0;
-  const int64_t parts = apply_values_splits(batch, N) + (R > 0 ? 1 : 0);
+  const int64_t parts = apply_values_splits(batch, N) + exact_splits(R);
   return parts > 1 ? (long long)(parts * batch * nq * D * (int64_t)sizeof(float)) : 0;
 }
 
@@ -442,7 +478,9 @@ static int apply_values(const float* w, long long w_bstride, long long w_qstride
   const int64_t n_splits = apply_values_splits(batch, N);
   const int64_t split_len = std::max<int64_t>(1, (N + n_splits - 1) / n_splits);
   const int64_t total = batch * nq * (int64_t)D;
-  const int64_t parts = n_splits + (R > 0 ? 1 : 0);
+  const int64_t x_splits = exact_splits(R), parts = n_splits + x_splits;
+  const int64_t groups = n_splits + x_splits * ((nq + kAvXQ - 1) / kAvXQ);
+  SMAQ_REQUIRE(groups < (1ll << 31), "smaq_cache_attend: %lld query rows by %lld exact rows are too many", nq, R);
   float* part = out;
   if (parts > 1) {
     SMAQ_REQUIRE(workspace && workspace_bytes >= parts * total * (int64_t)sizeof(float),
@@ -451,7 +489,7 @@ static int apply_values(const float* w, long long w_bstride, long long w_qstride
     part = (float*)workspace;
   }
   hipStream_t st = (hipStream_t)stream;
-  const dim3 grid((unsigned)parts, (unsigned)batch);
+  const dim3 grid((unsigned)groups, (unsigned)batch);
 #define SMAQ_AV(VPB, T)                                                                                           \
   hipLaunchKernelGGL((apply_values_kernel<VPB, T>), grid, dim3(kAvThreads), 0, st, w, (int64_t)w_bstride,          \
                      (int64_t)w_qstride, (int)nq, (int64_t)N, D, (const uint8_t*)data, (int64_t)d_bstride,           \

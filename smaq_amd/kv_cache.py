@@ -265,8 +265,15 @@ class SMAQKVCache:
         """Weights over [compressed, exact] applied to the dequantised and the
         exact values (smaq/kv_cache.py:243-267)."""
         h, ex = self._hist, self._exact
+        # One native call for a step's few query rows, and for more of them while
+        # the call is launches rather than work; past that a library product of
+        # the exact rows is the faster one.  us, one call / two products, 16 lanes
+        # of 8064 + 128 tokens: 1 row 22 / 67, 8 rows 35 / 66, 16 rows 86 / 67,
+        # 64 rows 324 / 314; 8064 + 4096: 4 rows 45 / 68, 8 rows 74 / 72, 64 rows
+        # 431 / 303; one lane, 8064 + 4096: 16 rows 50 / 67, 64 rows 180 / 195.
         if (h is not None and h.n and type(attn_weights) is torch.Tensor and attn_weights.is_cuda
-                and attn_weights.dtype == torch.float32 and attn_weights.is_contiguous()
+                and attn_weights.dtype == torch.float32 and attn_weights.is_contiguous() and attn_weights.dim() >= 2
+                and (attn_weights.shape[-2] <= 4 or attn_weights.numel() <= 1 << 20)
                 and attn_weights.device == h._bufs["v_data"].device and attn_weights.shape[:-2] == self._lead
                 and attn_weights.shape[-1] == h.n + ex.size and attn_weights.numel() and not _differentiated(attn_weights)
                 and self.head_dim in (32, 64, 128, 256) and self._exact_rows(ex.v, torch.float32)

@@ -18,6 +18,7 @@ import pytest
 import torch
 
 import smaq_amd as S
+from smaq_amd.value_codec import dequantize_values
 from oracle import smaq_ref as R
 from tests.conftest import sample_keys
 from tests.test_gpu_codecs import _ties_ok
@@ -175,3 +176,25 @@ def test_kv_cache_one_call_matches_the_general_path(dev, bits, vbits, dtype, lea
         w = torch.softmax(got, dim=-1)
         a, b = cache.attend(w), cache.attend(w.clone().requires_grad_()).detach()
         assert a.shape == b.shape and float((a - b).abs().max()) <= 2e-5 * float(b.abs().max())
+
+
+@pytest.mark.parametrize("D,vbits,lead,nq,N,R", [(128, 2, (2, 3), 9, 300, 257), (128, 2, (1, 1), 1, 33, 4096), (64, 4, (3,), 70, 129, 300),
+                                                 (32, 2, (), 8, 1000, 1), (256, 8, (2,), 17, 64, 513), (128, 4, (1, 2), 300, 70, 1030),
+                                                 (128, 2, (1,), 7, 40, 255)])
+def test_attend_long_windows_and_many_rows(dev, D, vbits, lead, nq, N, R):
+    """The exact window's rows and query rows over several workgroups: tiles of
+    query rows and splits of window rows, with remainders.  Each side is an fp32
+    sum of N + R products in an order of its own: 2e-5 of the largest result."""
+    cache = S.SMAQKVCache(D, value_bits=vbits, buffer_size=R, device=dev)
+    gen = torch.Generator().manual_seed(N + R)
+    k, v = (torch.randn(*lead, N + R, D, generator=gen).to(dev) for _ in range(2))
+    cache.prefill(k, v)
+    assert cache._exact.size == R
+    w = torch.softmax(2 * torch.randn(*lead, nq, N + R, generator=gen).to(dev), dim=-1)
+    got, want = cache.attend(w), cache.attend(w.clone().requires_grad_()).detach()
+    exact = (torch.matmul(w[..., :N].double(), dequantize_values(cache.value_quantized, 32).double())
+             + torch.matmul(w[..., N:].double(), v[..., N:, :].double()))
+    top = float(exact.abs().max())
+    assert got.shape == want.shape
+    assert float((got - want).abs().max()) <= 2e-5 * top and float((got.double() - exact).abs().max()) <= 2e-5 * top
+    assert torch.equal(got, cache.attend(w))
