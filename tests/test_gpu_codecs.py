@@ -500,6 +500,7 @@ def _encode_2d(dev, k, E, C, listed: bool):
     rc = N.lib().smaq_encode_blockvq_ws(N._ptr(k), N.dtype_code(k.dtype), 1, n, 0, k.stride(0), 0, nb, 2, nc, N._ptr(E),
                                         N._ptr(C), N._ptr(idx), ties.ptr(), N._ptr(ws), size, N._stream(dev))
     assert rc == 0
+    assert not listed or bool((ws != 0xA5).any())   # (the lists were built)
     return idx, ties.value()
 
 
@@ -545,6 +546,31 @@ def test_blockvq_2d_lists_match_the_scan(dev, nc, dtype, rows, shape):
     bad = (got != want).sum().item()
     assert bad == 0, f"{bad} of {want.numel()} indices differ"
     assert got_ties == ties
+
+
+@pytest.mark.parametrize("dtype,nb", [(torch.float16, 64), (torch.float32, 20)])
+def test_blockvq_2d_lists_in_columns(dev, dtype, nb):
+    """Rows of one head of three sequences into columns with room between them,
+    enough for more than 8 chunks of rows: indices and tie count of the scan,
+    and nothing written elsewhere."""
+    from smaq_amd import _native as N
+    g = torch.Generator().manual_seed(nb)
+    outer, inner, cap, nc = 3, 6001, 6144, 256
+    C, E = torch.randn(nb, nc, 2, generator=g), torch.eye(2).repeat(nb, 1, 1) + 0.2 * torch.randn(nb, 2, 2, generator=g)
+    C, E = C.to(dev), E.contiguous().to(dev)
+    heads = torch.randn(outer, inner, 2, 2 * nb, generator=g).to(dtype).to(dev)
+    k, got = heads[:, :, 1], []
+    for size in (0, N.lib().smaq_encode_blockvq_workspace_bytes(nb, 2, nc)):
+        idx = torch.full((outer, cap, nb), 255, dtype=torch.uint8, device=dev)
+        ws = torch.full((size,), 0xA5, dtype=torch.uint8, device=dev) if size else None
+        ties = N.TieCounter(dev)
+        rc = N.lib().smaq_encode_blockvq_ws(k.data_ptr(), N.dtype_code(dtype), outer, inner, k.stride(0), k.stride(1), cap,
+                                            nb, 2, nc, N._ptr(E), N._ptr(C), N._ptr(idx), ties.ptr(), N._ptr(ws), size,
+                                            N._stream(dev))
+        assert rc == 0 and (ws is None or bool((ws != 0xA5).any()))
+        assert bool((idx[:, inner:] == 255).all())
+        got.append((idx, ties.value()))
+    assert torch.equal(got[0][0], got[1][0]) and got[0][1] == got[1][1]
 
 
 @pytest.mark.parametrize("nb", [16, 12, 5])

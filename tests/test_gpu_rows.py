@@ -13,6 +13,7 @@ import torch
 
 import smaq_amd as S
 from smaq_amd.batch import PagedQuantizedKV, QuantizedKVBatch
+from smaq_amd.score import plan_hybrid_attention
 from tests.conftest import sample_keys
 
 pytestmark = pytest.mark.gpu
@@ -26,6 +27,16 @@ def _strategy(dev, codec, size, seed=0):
     x = sample_keys(nc, seed=seed + 6).reshape(nc, 128 // size, size).transpose(0, 1).contiguous().to(dev)
     strat.quantizer.load_state_dict({**strat.quantizer.state_dict(), "centroids": x, "decoded_centroids": x})
     return strat
+
+
+def _takes_rows(plan, q, got):
+    """Whether ``got`` is the row kernel's: without arrival counters the same
+    plan runs the kernels it would otherwise run, whose bits repeat."""
+    arrivals, plan.params.arrivals = plan.params.arrivals, None
+    other = plan.run(q).view_as(got).clone()
+    again = torch.equal(plan.run(q).view_as(got), other)
+    plan.params.arrivals = arrivals
+    return again and not torch.equal(other, got)
 
 
 def _close(got, ref, vals, what):
@@ -59,6 +70,7 @@ def test_rows_store_edges(dev, codec, size, vbits, g, T, dtype):
         _close(got, ref, (v,) if kr is None else (v, kr), f"{codec}{size} v{vbits} g{g} T{T} n{n} r{rn}")
         again = S.compute_hybrid_attention(q, st, kr, kr, 2 * g, query_positions=pos)
         assert torch.equal(got, again)
+        assert _takes_rows(plan_hybrid_attention(q, st, kr, kr, 2 * g, query_positions=pos), q.unsqueeze(0), got), (n, rn)
 
 
 @pytest.mark.parametrize("codec,size,vbits,g,T,dtype", FORMS[:7:3] + FORMS[4:5])
@@ -89,8 +101,9 @@ def test_rows_ragged_batches(dev, codec, size, vbits, g, T, dtype, block_size):
         for p in plans:
             if cut is not None:
                 p.set_lengths(hist_len=cut)
-        got, ref = (p.run(q) for p in plans)
+        got, ref = (p.run(q).clone() for p in plans)
         _close(got, ref, vals, f"{codec}{size} v{vbits} g{g} T{T} block {block_size} {'cut' if cut is not None else ''}")
+        assert _takes_rows(plans[0], q, got)
         assert not plans[0].arrivals.any()
 
 
