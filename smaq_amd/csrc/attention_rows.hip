@@ -21,7 +21,10 @@ __global__ __launch_bounds__(256) void rows_combine_kernel(smaq_attn_params p, R
                 ti, tid, nullptr);
 }
 
-// query tokens below the prefill kernel's own range
+// query tokens: chunks of 64 and more are the prefill kernel's, the automatic
+// choice for them being what an explicit impl 3 runs (callers compare the two
+// bit for bit), although this kernel is the faster one beyond (30000 tokens,
+// 32/8 heads, prefill / this kernel, us: 64 tokens 389 / 213, 128 427 / 386)
 constexpr int kRowsMaxT = 63;
 
 bool rows_supported(const smaq_attn_params& p) {
@@ -49,17 +52,23 @@ bool rows_supported(const smaq_attn_params& p) {
 // From 16 query tokens on the prefill kernel serves the call as well.  It
 // decodes every key once into tile images and takes 256 query rows of one head
 // at a time, mostly empty ones for a short chunk; this kernel decodes a key
-// once per 8 rows.  Times over tokens x KV heads of history (MI355X, whole
-// plan): this kernel 25.5 ps per tile of 8 rows, prefill 0.46 ns and 0.22 ns
-// per query head, and about 20 us and 0.25 us per query token more beside
-// them.  30000 tokens (prefill / this kernel, us): 32/8 heads T = 16 373 / 80,
-// 32 372 / 123, 64 389 / 213, 128 427 / 386; 28/4 heads T = 32 318 / 114; 4000
-// tokens, 28/4 heads, T = 16 94 / 37, 32 98 / 48.  From kRowsMaxT tokens on the
-// choice is the prefill kernel's, as callers of such chunks know it.
+// once per 8 rows, and the window beside it goes through the recent window's
+// kernel, once per 8 rows and without the matrix cores.  Times over tokens x KV
+// heads (MI355X, whole plan; fitted to 500 to 30000 tokens of history, windows
+// of 0 to 16384, 16 to 63 query tokens, 32/8 and 28/4 heads): history 23.6 ps
+// per tile of 8 rows here, 0.42 ns and 0.18 ns per query head there; window
+// 128 ps per tile here, 0.12 ns and 0.38 ns per query head there; the prefill
+// kernel 18 us more beside them, and 15 us with a window.  Prefill / this
+// kernel, us: 30000 tokens, 32/8 heads, T = 16 344 / 75, 63 363 / 208; with a
+// window of 4096 T = 63 448 / 343, of 16384 623 / 728; 500 tokens, T = 63,
+// windows of 128, 1024, 4096 76 / 36, 88 / 81, 127 / 164.
 bool rows_preferred(const smaq_attn_params& p) {
   const double g = p.n_q_heads / p.n_kv_heads, tiles = (double)((p.q_len * (p.n_q_heads / p.n_kv_heads) + kRowsQ - 1) / kRowsQ);
-  const double tokens = (double)p.batch * p.n_kv_heads * (double)p.max_hist_len;
-  return tokens * (0.0255 * tiles - 0.46 - 0.22 * g) * 1e-3 < 20.0 + 0.25 * p.q_len;
+  const double heads = (double)p.batch * p.n_kv_heads * 1e-3;
+  const double window = p.has_recent && p.max_recent_len > 0 ? (double)p.max_recent_len : 0.0;
+  return heads * (double)p.max_hist_len * (0.0236 * tiles - 0.42 - 0.18 * g) +
+             heads * window * (0.128 * tiles - 0.12 - 0.38 * g) <
+         18.0 + (window > 0.0 ? 15.0 : 0.0);
 }
 
 // Workgroups of the grid: what the device holds at once.

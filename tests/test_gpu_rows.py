@@ -312,3 +312,21 @@ def test_rows_past_the_built_in_scratch(dev):
     plan.out.fill_(float("nan"))
     _native.attn_hybrid_noalloc(plan.params, dev)
     assert torch.equal(plan.out, ref)
+
+
+@pytest.mark.parametrize("codec,size", [("vq", 8), ("scalar", 3)])
+@pytest.mark.parametrize("T,n,rn,prefill", [(63, 500, 4096, True), (63, 500, 128, False), (63, 30000, 4096, False),
+                                            (16, 500, 4096, False), (32, 500, 16384, True)])
+def test_rows_long_window_chunks(dev, codec, size, T, n, rn, prefill):
+    """Chunks beside a long exact window: the window's cost counts in the
+    choice between the row and the prefill kernel."""
+    strat = _strategy(dev, codec, size)
+    st = S.CompressedKVStore(128, 4, device=dev, key_strategy=strat)
+    k = sample_keys(n * 4, seed=n).view(n, 4, 128).bfloat16().to(dev)
+    st.append_chunk(k, k)
+    q = sample_keys(T * 28, seed=T).view(T, 28, 128).to(dev)
+    kr = sample_keys(rn * 4, seed=rn).view(rn, 4, 128).bfloat16().to(dev)
+    pos = torch.arange(n + rn - T, n + rn, device=dev)
+    got, big, ref = (S.compute_hybrid_attention(q, st, kr, kr, 28, query_positions=pos, impl=i) for i in (0, 3, 1))
+    assert torch.equal(got, big) == prefill
+    _close(got, ref, (k, kr), f"{codec}{size} T{T} n{n} r{rn}")
