@@ -449,7 +449,7 @@ extern "C" int smaq_cache_attend(const float* w, long long w_bstride, long long 
                                  int group, const void* scales, const void* zeros, long long s_bstride, int sdtype,
                                  long long R, const float* xv, long long xv_bstride, float* out, void* workspace,
                                  long long workspace_bytes, void* stream) {
-  SMAQ_REQUIRE(R >= 0 && (R == 0 || xv), "smaq_cache_attend: exact rows without a pointer");
+  SMAQ_REQUIRE(R >= 0 && (R == 0 || (xv && w)), "smaq_cache_attend: exact rows or their weights without a pointer");
   return apply_values(w, w_bstride, w_qstride, batch, nq, N, D, data, d_bstride, bits, group, scales, zeros, s_bstride,
                       sdtype, R, xv, xv_bstride, out, workspace, workspace_bytes, stream);
 }

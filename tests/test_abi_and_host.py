@@ -60,6 +60,15 @@ def test_status_codes_map_to_exceptions():
     assert lib.smaq_attn_hybrid(ctypes.byref(p), None) == -1
 
 
+def test_cache_attend_rejects_exact_rows_without_weights():
+    """(an empty history asks for no weights of its own): an error of the call,
+    with nothing launched."""
+    lib = _native.lib()
+    d = ctypes.c_void_p(256)
+    st = lib.smaq_cache_attend(None, 5, 5, 1, 1, 0, 128, None, 0, 2, 32, None, None, 0, 0, 5, d, 640, d, d, 1 << 20, None)
+    assert st == -1 and b"without a pointer" in lib.smaq_last_error()
+
+
 def test_attn_workspace_size():
     p = _native.AttnParams()
     p.batch, p.q_len, p.n_q_heads, p.n_kv_heads, p.head_dim = 32, 1, 32, 8, 128
