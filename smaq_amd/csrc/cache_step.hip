@@ -174,6 +174,12 @@ extern "C" int smaq_cache_scores(const void* q, int qdtype, long long batch, lon
                "smaq_cache_scores: bad shape");
   SMAQ_REQUIRE((((uintptr_t)M | (uintptr_t)codes | (uintptr_t)codes_bstride) & 15) == 0,
                "smaq_cache_scores: the metric and the code rows must be 16-byte aligned");
+  auto known = [](int t) { return t == SMAQ_F32 || t == SMAQ_F16 || t == SMAQ_BF16; };
+  if (!known(qdtype) || !known(ndtype)) {
+    set_error("smaq_cache_scores: unsupported %s dtype %d", known(qdtype) ? "norm" : "query",
+              known(qdtype) ? ndtype : qdtype);
+    return SMAQ_EUNSUPPORTED;
+  }
   hipStream_t st = (hipStream_t)stream;
   const int64_t rows = (int64_t)batch * nq;
   hipLaunchKernelGGL(cache_rotate_kernel, dim3((unsigned)((rows + kCsRows - 1) / kCsRows)), dim3(256), 0, st, q, qdtype,
@@ -187,14 +193,12 @@ extern "C" int smaq_cache_scores(const void* q, int qdtype, long long batch, lon
   switch (ndtype) {                                                                                    \
     case SMAQ_F32: SMAQ_CS(float, T); break;                                                           \
     case SMAQ_F16: SMAQ_CS(_Float16, T); break;                                                        \
-    case SMAQ_BF16: SMAQ_CS(bf16, T); break;                                                           \
-    default: set_error("smaq_cache_scores: unsupported norm dtype %d", ndtype); return SMAQ_EUNSUPPORTED; \
+    default: SMAQ_CS(bf16, T); break;                                                                  \
   }
   switch (qdtype) {
     case SMAQ_F32: SMAQ_CS_N(float) break;
     case SMAQ_F16: SMAQ_CS_N(_Float16) break;
-    case SMAQ_BF16: SMAQ_CS_N(bf16) break;
-    default: set_error("smaq_cache_scores: unsupported query dtype %d", qdtype); return SMAQ_EUNSUPPORTED;
+    default: SMAQ_CS_N(bf16) break;
   }
 #undef SMAQ_CS_N
 #undef SMAQ_CS

@@ -69,6 +69,14 @@ def test_cache_attend_rejects_exact_rows_without_weights():
     assert st == -1 and b"without a pointer" in lib.smaq_last_error()
 
 
+@pytest.mark.parametrize("qdtype,ndtype", [(9, 0), (0, 9)])
+def test_cache_scores_rejects_unknown_dtypes_before_any_launch(qdtype, ndtype):
+    lib = _native.lib()
+    d = ctypes.c_void_p(256)
+    st = lib.smaq_cache_scores(d, qdtype, 1, 1, 128, d, d, 4, d, 256, 3, d, 4, ndtype, d, 0, None, 0, 1.0, d, None)
+    assert st == -2 and b"dtype 9" in lib.smaq_last_error()
+
+
 def test_attn_workspace_size():
     p = _native.AttnParams()
     p.batch, p.q_len, p.n_q_heads, p.n_kv_heads, p.head_dim = 32, 1, 32, 8, 128
