@@ -308,7 +308,9 @@ __global__ __launch_bounds__(kAvThreads) void apply_values_kernel(
     for (int q = 0; q < kAvQ; ++q)
 #pragma unroll
       for (int e = 0; e < DPL; ++e) acc[q][e] = 0.0f;
-#pragma unroll 4
+    // (four rows in flight take 176 registers instead of 161, 2 workgroups a CU
+    // instead of 3: 64 lanes of 8064 tokens, 16 query rows 235 -> 311 us)
+#pragma unroll 2
     for (int64_t t = t0 + (int64_t)wv * tpw + tl; t < t1; t += 4 * tpw) {
       const uint32_t word = *(const uint32_t*)(dcol + t * row_bytes);
       const float sc = Num<T>::to_f(scol[t * ng]);
@@ -356,12 +358,18 @@ __global__ __launch_bounds__(256) void apply_values_reduce_kernel(const float* _
   out[i] = acc;
 }
 
-// token splits of a launch: at least 256 tokens each (2 x 8 heads x 8064
-// tokens, one query row: 17.4 + 4.7 us with 512 tokens; 16.6 + 3.8 with the
-// exact rows as a split of their own), about 2048 workgroups
-static int64_t apply_values_splits(long long batch, long long N) {
-  const int64_t by_len = std::max<int64_t>(1, (N + 255) / 256);
-  const int64_t by_grid = std::max<int64_t>(1, (2048 + batch - 1) / std::max<long long>(1, batch));
+// Token splits of a launch: 256 tokens each while those fit one round of the
+// device (3 workgroups a CU), else at least 512 tokens and about 2048
+// workgroups.  Whole call, us, 512 / 256 tokens: 16 lanes of 8064, 1 query row
+// 20 (the host) / 20, 16 rows 77 / 60; 16 of 16384 (1024 workgroups of 256)
+// 23 / 29, 64 of 4096 20 / 28.  Up to 512 tokens and 4 query rows one split,
+// which needs no second launch: 300 tokens 16 / 20 (16 rows 44 / 33).
+static int64_t apply_values_splits(long long batch, long long nq, long long N) {
+  const int64_t lanes = std::max<long long>(1, batch), fine = std::max<int64_t>(1, (N + 255) / 256);
+  if (N <= 512 && nq <= kAvQ) return 1;
+  if (fine <= 768 / lanes) return fine;
+  const int64_t by_len = std::max<int64_t>(1, (N + 511) / 512);
+  const int64_t by_grid = std::max<int64_t>(1, (2048 + lanes - 1) / lanes);
   return std::min<int64_t>(std::min(by_len, by_grid), 65535);
 }
 
@@ -418,7 +426,7 @@ extern "C" int smaq_dequant_values(const void* data, const void* scales, const v
 
 extern "C" long long smaq_apply_values_workspace_bytes(long long batch, long long nq, long long N, int D) {
   if (batch <= 0 || nq <= 0 || D <= 0) return 0;
-  const int64_t n_splits = apply_values_splits(batch, N);
+  const int64_t n_splits = apply_values_splits(batch, nq, N);
   return n_splits > 1 ? (long long)(n_splits * batch * nq * D * (int64_t)sizeof(float)) : 0;
 }
 
@@ -440,7 +448,7 @@ extern "C" int smaq_apply_values(const float* w, long long w_bstride, long long 
 
 extern "C" long long smaq_cache_attend_workspace_bytes(long long batch, long long nq, long long N, long long R, int D) {
   if (batch <= 0 || nq <= 0 || D <= 0) return 0;
-  const int64_t parts = apply_values_splits(batch, N) + exact_splits(R);
+  const int64_t parts = apply_values_splits(batch, nq, N) + exact_splits(R);
   return parts > 1 ? (long long)(parts * batch * nq * D * (int64_t)sizeof(float)) : 0;
 }
 
@@ -475,7 +483,7 @@ static int apply_values(const float* w, long long w_bstride, long long w_qstride
     return SMAQ_EUNSUPPORTED;
   }
   SMAQ_REQUIRE(((uintptr_t)data % 4) == 0 && d_bstride % 4 == 0, "smaq_apply_values: value rows must be 4-byte aligned");
-  const int64_t n_splits = apply_values_splits(batch, N);
+  const int64_t n_splits = apply_values_splits(batch, nq, N);
   const int64_t split_len = std::max<int64_t>(1, (N + n_splits - 1) / n_splits);
   const int64_t total = batch * nq * (int64_t)D;
   const int64_t x_splits = exact_splits(R), parts = n_splits + x_splits;

@@ -69,6 +69,15 @@ def test_cache_attend_rejects_exact_rows_without_weights():
     assert st == -1 and b"without a pointer" in lib.smaq_last_error()
 
 
+@pytest.mark.parametrize("lanes,nq,n,splits", [(16, 1, 300, 1), (16, 5, 300, 2), (16, 1, 513, 3), (16, 1, 8064, 32), (24, 1, 8064, 32),
+                                               (25, 1, 8064, 16), (16, 1, 16384, 32), (64, 16, 4096, 8), (64, 1, 32768, 32),
+                                               (1, 1, 200000, 391), (1, 16, 196608, 768)])
+def test_apply_values_token_splits(lanes, nq, n, splits):
+    """256 tokens a split while those are one round of workgroups, 512 beyond."""
+    need = _native.lib().smaq_apply_values_workspace_bytes(lanes, nq, n, 128)
+    assert need == (splits * lanes * nq * 128 * 4 if splits > 1 else 0)
+
+
 @pytest.mark.parametrize("qdtype,ndtype", [(9, 0), (0, 9)])
 def test_cache_scores_rejects_unknown_dtypes_before_any_launch(qdtype, ndtype):
     lib = _native.lib()
