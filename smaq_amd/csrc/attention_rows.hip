@@ -1,5 +1,7 @@
 // Scalar-key instances of the matrix-core row kernel (attention_rows.h) and
 // the rule that says which calls take it.
+#include <algorithm>
+
 #include "attention_rows.h"
 
 namespace smaq {
@@ -79,9 +81,14 @@ static RowsRule rows_rule(const smaq_attn_params& p, int n_recent) {
   const bool scalar = p.key_format == SMAQ_KEY_SCALAR;
   r.groups = device_cu_count() * (scalar ? 2 : 1);
   // A share of at least 512 tokens: a piece costs a partial and a load in the
-  // merge (5 query tokens over 4001, whole call: shares from 128 / 256 / 512
-  // tokens 177 / 155 / 148 us).
-  r.least = scalar ? 4 : 2;
+  // merge (5 query tokens over 4001 and a window of 100, 4-bit keys and values,
+  // whole call: shares from 128 / 256 / 512 / 1024 tokens 37.3 / 35.4 / 33.5 /
+  // 37.6 us; 8-dim block-VQ keys from 256 / 512 / 1024 tokens 37.4 / 35.7 / 38.1).
+  // But never several units that are whole each: 16 sequences of 16 tokens, 16
+  // query tokens at 8/8 heads, 38.6 us with four units a share.
+  const int step = kRowsTile * (scalar ? RowsKey<0>::kWaves : RowsKey<8>::kWaves);
+  const int64_t steps = (p.max_hist_len + step - 1) / step;
+  r.least = (int)std::min<int64_t>(scalar ? 4 : 2, steps);
   r.n_recent = n_recent;
   return r;
 }

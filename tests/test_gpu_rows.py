@@ -330,3 +330,25 @@ def test_rows_long_window_chunks(dev, codec, size, T, n, rn, prefill):
     got, big, ref = (S.compute_hybrid_attention(q, st, kr, kr, 28, query_positions=pos, impl=i) for i in (0, 3, 1))
     assert torch.equal(got, big) == prefill
     _close(got, ref, (k, kr), f"{codec}{size} T{T} n{n} r{rn}")
+
+
+@pytest.mark.parametrize("codec,size", [("scalar", 3), ("vq", 2), ("vq", 8)])
+@pytest.mark.parametrize("n", [1, 31, 128, 129, 257, 513])
+def test_rows_shares_of_whole_units(dev, codec, size, n):
+    """Histories below the least share: a unit a share, whole; above it, in
+    pieces; lengths that differ included."""
+    strat = _strategy(dev, codec, size)
+    B, h, g, T = 5, 2, 2, 7
+    k = sample_keys(B * n * h, seed=1).view(B, n, h, 128).to(dev)
+    kv = QuantizedKVBatch.encode(strat, k, k)
+    q = sample_keys(B * T * h * g, seed=2).view(B, T, h * g, 128).to(dev)
+    plans = [kv.plan(q, impl=i) for i in (0, 1)]
+    for cut in (None, [n, 0, 1, max(n - 1, 0), n // 2]):
+        if cut is not None and plans[0].hist_len is None:
+            continue
+        for p in plans:
+            if cut is not None:
+                p.set_lengths(hist_len=torch.tensor(cut, device=dev))
+        got, ref = (p.run(q).clone() for p in plans)
+        _close(got, ref, (k,), f"{codec}{size} n{n} {cut}")
+        assert torch.equal(got, plans[0].run(q))
