@@ -330,8 +330,8 @@ typedef struct smaq_attn_params {
      head_dim 128: the decode kernel for single-token queries it serves; with
      arrival counters (below), block-VQ or 3/4-bit scalar keys and 2- or
      4-bit values in groups of 32, the matrix-core row kernel for other
-     decode shapes and for fewer than 64 query tokens (from 16 on where it is
-     the faster one); the prefill kernel for q_len >= 16; the generic kernels
+     decode shapes and for fewer than 64 query tokens, where it is estimated to
+     be the faster one; the prefill kernel for q_len >= 16; the generic kernels
      otherwise. */
   int impl;
   /* Optional split merge inside the matrix-core decode kernel (NULL: a

@@ -493,12 +493,9 @@ static Plan make_plan(const smaq_attn_params* p, bool allow_rows) {
   pl.prefill = (p->impl == 0 || p->impl == 3) && !pl.mfma && prefill_mfma_supported(*p);
   // The row kernel merges the recent window's partials and leaves none of its
   // own for a combine, so with a window it takes complete calls only: calls
-  // that share a workspace phase by phase agree on the generic layout.  It wins wherever it is supported: 37x at 16 x 32768
-  // tokens, 43x at 64 paged sequences (attention_rows.h), 12x for the whole
-  // call at 5 query tokens over 4001, and down to 16 tokens (28/4 heads, plan
-  // alone: 33 against 46 us of scalar keys, 23 against 37 of block-VQ).
+  // that share a workspace phase by phase agree on the generic layout.
   const int phase_mask = p->phases ? p->phases : 15;
-  pl.rows = allow_rows && !pl.mfma && rows_supported(*p) && (!pl.prefill || rows_preferred(*p)) &&
+  pl.rows = allow_rows && !pl.mfma && rows_supported(*p) && rows_preferred(*p, pl.prefill) &&
             (!p->has_recent || p->max_recent_len <= 0 || (phase_mask & 7) == 7);
   if (pl.rows) pl.prefill = false;
   const int64_t units = (int64_t)p->batch * p->n_kv_heads * pl.row_tiles;

@@ -151,8 +151,9 @@ int launch_mfma_decode(const smaq_attn_params& p, const HistAddr& a, const Parti
 // workspace; the `n_recent` partials per row of `recent` (written by the
 // recent launch of the same call) are merged in.
 bool rows_supported(const smaq_attn_params& p);
-// whether it is the faster kernel where the prefill kernel serves the call too
-bool rows_preferred(const smaq_attn_params& p);
+// whether it is faster than the kernel the call takes otherwise (`prefill`: the
+// prefill kernel, else the generic ones)
+bool rows_preferred(const smaq_attn_params& p, bool prefill);
 int64_t rows_bytes(const smaq_attn_params& p);
 int launch_rows(const smaq_attn_params& p, const HistAddr& a, void* slots, const Partials& recent, int n_recent,
                 hipStream_t st);

@@ -51,26 +51,47 @@ bool rows_supported(const smaq_attn_params& p) {
   return !p.block_table || (p.block_size >= 16 && (p.block_size & (p.block_size - 1)) == 0);
 }
 
-// From 16 query tokens on the prefill kernel serves the call as well.  It
-// decodes every key once into tile images and takes 256 query rows of one head
-// at a time, mostly empty ones for a short chunk; this kernel decodes a key
-// once per 8 rows, and the window beside it goes through the recent window's
-// kernel, once per 8 rows and without the matrix cores.  Times over tokens x KV
-// heads (MI355X, whole plan; fitted to 500 to 30000 tokens of history, windows
-// of 0 to 16384, 16 to 63 query tokens, 32/8 and 28/4 heads): history 23.6 ps
-// per tile of 8 rows here, 0.42 ns and 0.18 ns per query head there; window
-// 128 ps per tile here, 0.12 ns and 0.38 ns per query head there; the prefill
-// kernel 18 us more beside them, and 15 us with a window.  Prefill / this
-// kernel, us: 30000 tokens, 32/8 heads, T = 16 344 / 75, 63 363 / 208; with a
-// window of 4096 T = 63 448 / 343, of 16384 623 / 728; 500 tokens, T = 63,
-// windows of 128, 1024, 4096 76 / 36, 88 / 81, 127 / 164.
-bool rows_preferred(const smaq_attn_params& p) {
-  const double g = p.n_q_heads / p.n_kv_heads, tiles = (double)((p.q_len * (p.n_q_heads / p.n_kv_heads) + kRowsQ - 1) / kRowsQ);
-  const double heads = (double)p.batch * p.n_kv_heads * 1e-3;
+// Whether this kernel is the faster one, by estimated times in us over units of
+// (sequence, KV head), tiles of 8 query rows here and of 16 in the generic
+// kernels.  MI355X, whole plan, fitted to 4600 calls (1 to 800 sequences of 16 to
+// 30000 tokens, 1 to 63 query tokens, windows of 0 to 16384, 28/4, 32/8 and 8/8
+// heads): of the calls that differ by more than 2 us, 68 take the slower kernel,
+// by 20% at most.
+//
+// A unit costs this kernel a chain of round trips whatever its length.
+//   Below 16 query tokens the generic kernels are ahead for many sequences of a
+// few tokens with block-VQ keys (one workgroup of 8 waves a CU here), where the
+// rows fill several tiles badly or a window makes the unit leave a partial: 512
+// sequences of 16 tokens, 3 query tokens at 32/8 heads, 8-dim blocks, 293 us here,
+// 217 there; of 100 tokens 310 and 430.
+//   From 16 query tokens on the prefill kernel serves the call.  It decodes every
+// key once into tile images and takes 256 query rows of one head at a time,
+// mostly empty ones for a short chunk, where this kernel decodes a key once per
+// tile, and the window beside it goes through the recent window's kernel, once
+// per tile and without the matrix cores.  Prefill / this kernel: 30000 tokens,
+// 32/8 heads, T = 16 344 / 75, 63 363 / 208; with a window of 4096 T = 63
+// 448 / 343, of 16384 623 / 728; 500 tokens, T = 63, windows of 128, 1024, 4096
+// 76 / 36, 88 / 81, 127 / 164; 512 sequences of 16 and 300 tokens of 8-dim
+// block-VQ keys, T = 24, 28/4 heads 888 / 1586 and 1858 / 2008.
+bool rows_preferred(const smaq_attn_params& p, bool prefill) {
+  const bool scalar = p.key_format == SMAQ_KEY_SCALAR;
+  const int g = p.n_q_heads / p.n_kv_heads, rows = p.q_len * g, tiles = (rows + kRowsQ - 1) / kRowsQ;
+  const double units = (double)p.batch * p.n_kv_heads, hist = (double)p.max_hist_len;
   const double window = p.has_recent && p.max_recent_len > 0 ? (double)p.max_recent_len : 0.0;
-  return heads * (double)p.max_hist_len * (0.0236 * tiles - 0.42 - 0.18 * g) +
-             heads * window * (0.128 * tiles - 0.12 - 0.38 * g) <
-         18.0 + (window > 0.0 ? 15.0 : 0.0);
+  if (!prefill) {
+    if (scalar || (tiles == 1 && window == 0.0)) return true;
+    const double blocks = 128.0 / p.vq_block_dim, halves = (rows + 15) / 16;
+    const double here = 8.4 + units * (tiles * (0.0323 + 20e-6 * hist) + (tiles > 1 ? 0.0085 : 0.0154));
+    const double there = 22.8 + units * (halves * (0.0103 + 0.13e-3 * blocks + (1.08e-3 + 4.6e-6 * blocks) * hist) + 0.0018 * rows);
+    return here <= there;
+  }
+  const bool split = prefill_split_len(p, p.max_hist_len) < p.max_hist_len;  // (a combine launch)
+  const double here = 14.5 + (window > 0.0 ? 9.0 : 0.0) +
+                      units * tiles * ((scalar ? 0.0184 : 0.0369) + 26e-6 * hist + 0.148e-3 * window);
+  const double there = 20.2 + (split ? 8.0 : 0.0) + (window > 0.0 ? 21.9 : 0.0) +
+                       units * (g * (0.0216 + 1.24e-3 * p.q_len + 0.217e-3 * hist + 0.358e-3 * window) +
+                                0.011 + 0.478e-3 * hist + 0.64e-3 * window);
+  return here <= there;
 }
 
 // Workgroups of the grid: what the device holds at once.

@@ -332,6 +332,24 @@ def test_rows_long_window_chunks(dev, codec, size, T, n, rn, prefill):
     _close(got, ref, (k, kr), f"{codec}{size} T{T} n{n} r{rn}")
 
 
+@pytest.mark.parametrize("size,B,n,T,hq,h,rn,rows", [(8, 512, 16, 3, 32, 8, 0, False), (8, 512, 100, 3, 32, 8, 0, True),
+                                                      (8, 512, 16, 3, 8, 8, 0, True), (8, 200, 16, 3, 8, 8, 32, False),
+                                                      (2, 200, 16, 24, 28, 4, 0, False), (2, 200, 1000, 24, 28, 4, 0, True)])
+def test_rows_many_short_sequences(dev, size, B, n, T, hq, h, rn, rows):
+    """Many sequences of a few tokens, whose units the generic and prefill kernels
+    work through faster: without arrival counters, which the row kernel needs,
+    the same call gives the same bits where it did not run."""
+    strat = _strategy(dev, "vq", size)
+    k = sample_keys(B * n * h, seed=1).view(B, n, h, 128).bfloat16().to(dev)
+    kv = QuantizedKVBatch.encode(strat, k, k)
+    q = sample_keys(B * T * hq, seed=2).view(B, T, hq, 128).to(dev)
+    rk = sample_keys(B * rn * h, seed=3).view(B, rn, h, 128).bfloat16().to(dev) if rn else None
+    plan = kv.plan(q, None, rk, rk)
+    got = plan.run(q).clone()
+    _close(got, kv.plan(q, None, rk, rk, impl=1).run(q), (k,), f"vq{size} B{B} n{n} T{T} r{rn}")
+    assert _takes_rows(plan, q, got) == rows
+
+
 @pytest.mark.parametrize("codec,size", [("scalar", 3), ("vq", 2), ("vq", 8)])
 @pytest.mark.parametrize("n", [1, 31, 128, 129, 257, 513])
 def test_rows_shares_of_whole_units(dev, codec, size, n):
