@@ -39,13 +39,13 @@
 // The QK and PV products are accumulated in fp32 and carry ~22 bits of each
 // operand.
 //
-// What bounds it: VALU issue (341 per tile: 68% of the cycles at 16 x 32768
+// What bounds it: VALU issue (349 per tile: 71% of the cycles at 16 x 32768
 // tokens of 8-dim block-VQ keys).  Measured, whole call, before (generic
-// kernels) and now: that batch at 32/8 heads 4326 -> 116 us (2.3 TB/s of
+// kernels) and now: that batch at 32/8 heads 4326 -> 114 us (2.3 TB/s of
 // 64-byte rows), 64 paged sequences of up to 8000 tokens of 3-bit keys at
-// 28/4 heads 2906 -> 67 us (1.8 TB/s of 114-byte rows); its kernel alone over
+// 28/4 heads 2899 -> 68 us (1.8 TB/s of 114-byte rows); its kernel alone over
 // one sequence of 65408 tokens of 2-dim block-VQ keys at 28/4 heads 339 (and
-// 33 to combine) -> 32 us.
+// 33 to combine) -> 35 us.
 #pragma once
 
 #include "decode_common.h"

@@ -41,9 +41,12 @@
 // token l of the set in lane l, which forms the nearest quad's four distances
 // again from the LDS codebook (the same terms, v_dot2_f32_f16: at most 2^-23 S
 // for each of 13 steps, 1.6e-6) for the clear test, the index, the store and
-// the exact recount.  VALU bound (77 % of the busy cycles), with the LDS busy half of them; value
-// and index of every single distance took 30 % more VALU instructions:
-// 4,194,304 rows of 16 blocks, their value pack included, 2253 -> 2116 us.
+// the exact recount.  VALU bound (80 % of the busy cycles), with the LDS busy half
+// of them, most of that in conflicts of the quads' rows (3.1e8 of 4.8e8 cycles);
+// 56 bytes a lane of scratch (fp32 keys 100).  Value and index of every single
+// distance took 30 % more VALU instructions, no scratch and 5.5e7 cycles of
+// conflicts: 4,194,304 rows of 16 blocks, their value pack included, 2253 us
+// against 2116; keys alone, 524,288 rows 285 against 260 (fp32 318 against 290).
 #include "encode_internal.h"
 
 namespace smaq {

@@ -221,7 +221,7 @@ constexpr int kAvMaxD = 512;
 // A workgroup of the exact rows (smaq_cache_attend): kAvXRows of them for kAvXQ
 // query rows, so that a long window or many query rows fill the device (one
 // workgroup a lane for the whole window and every query row: 16 lanes of 8064
-// tokens, window 4096, one row 80 us, 8 rows 508, 64 rows 3985; now 29, 74, 431.
+// tokens, window 4096, one row 80 us, 8 rows 508, 64 rows 3985; now 21, 45, 327.
 // A row of a window of 128 as before, 17 us).
 constexpr int kAvXRows = 256;
 constexpr int kAvXQ = 8;

@@ -268,9 +268,10 @@ class SMAQKVCache:
         # One native call for a step's few query rows, and for more of them while
         # the call is launches rather than work; past that a library product of
         # the exact rows is the faster one.  us, one call / two products, 16 lanes
-        # of 8064 + 128 tokens: 1 row 22 / 67, 8 rows 35 / 66, 16 rows 86 / 67,
-        # 64 rows 324 / 314; 8064 + 4096: 4 rows 45 / 68, 8 rows 74 / 72, 64 rows
-        # 431 / 303; one lane, 8064 + 4096: 16 rows 50 / 67, 64 rows 180 / 195.
+        # of 8064 + 128 tokens: 1 row 17 / 69, 8 rows 31 / 70, 16 rows 80 / 69,
+        # 64 rows 296 / 296; 8064 + 4096: 4 rows 28 / 70, 8 rows 45 / 70, 16 rows
+        # 88 / 104, 64 rows 327 / 286; one lane, 8064 + 4096: 16 rows 48 / 70, 64
+        # rows 171 / 186.
         if (h is not None and h.n and type(attn_weights) is torch.Tensor and attn_weights.is_cuda
                 and attn_weights.dtype == torch.float32 and attn_weights.is_contiguous() and attn_weights.dim() >= 2
                 and (attn_weights.shape[-2] <= 4 or attn_weights.numel() <= 1 << 20)
