@@ -331,7 +331,7 @@ typedef struct smaq_attn_params {
      arrival counters (below), block-VQ or 3/4-bit scalar keys and 2- or
      4-bit values in groups of 32, the matrix-core row kernel for other
      decode shapes and for fewer than 64 query tokens, where it is estimated to
-     be the faster one; the prefill kernel for q_len >= 16; the generic kernels
+     be the faster one or, from 16 on, is the more exact one; the prefill kernel for q_len >= 16; the generic kernels
      otherwise. */
   int impl;
   /* Optional split merge inside the matrix-core decode kernel (NULL: a

@@ -1,6 +1,7 @@
 // Scalar-key instances of the matrix-core row kernel (attention_rows.h) and
 // the rule that says which calls take it.
 #include <algorithm>
+#include <cmath>
 
 #include "attention_rows.h"
 
@@ -53,10 +54,10 @@ bool rows_supported(const smaq_attn_params& p) {
 
 // Whether this kernel is the faster one, by estimated times in us over units of
 // (sequence, KV head), tiles of 8 query rows here and of 16 in the generic
-// kernels.  MI355X, whole plan, fitted to 4600 calls (1 to 800 sequences of 16 to
+// kernels.  MI355X, whole plan, fitted to 5400 calls (1 to 800 sequences of 16 to
 // 30000 tokens, 1 to 63 query tokens, windows of 0 to 16384, 28/4, 32/8 and 8/8
-// heads): of the calls that differ by more than 2 us, 68 take the slower kernel,
-// by 20% at most.
+// heads): of the calls in bf16 that differ by more than 4% and 2 us, 84 take the
+// slower kernel, by 21% at most.
 //
 // A unit costs this kernel a chain of round trips whatever its length.
 //   Below 16 query tokens the generic kernels are ahead for many sequences of a
@@ -86,8 +87,14 @@ bool rows_preferred(const smaq_attn_params& p, bool prefill) {
     return here <= there;
   }
   const bool split = prefill_split_len(p, p.max_hist_len) < p.max_hist_len;  // (a combine launch)
+  // Only where its values are as exact in f16 as here: 2-bit codes with bf16 scales
+  // and no fp32 window (error beside the generic kernels: 1e-7 to 1e-6 both; fp32
+  // or fp16 scales or 4-bit codes 1e-5 to 2e-4 there).
+  if (p.val_bits != 2 || p.val_dtype != SMAQ_BF16 || (window > 0.0 && p.recent_dtype == SMAQ_F32)) return true;
+  // (the window's kernel takes chunks of 64 tokens)
+  const double chunks = std::ceil(window / 64.0) * 9.5e-3;
   const double here = 14.5 + (window > 0.0 ? 9.0 : 0.0) +
-                      units * tiles * ((scalar ? 0.0184 : 0.0369) + 26e-6 * hist + 0.148e-3 * window);
+                      units * tiles * ((scalar ? 0.0184 : 0.0369) + 26e-6 * hist + chunks);
   const double there = 20.2 + (split ? 8.0 : 0.0) + (window > 0.0 ? 21.9 : 0.0) +
                        units * (g * (0.0216 + 1.24e-3 * p.q_len + 0.217e-3 * hist + 0.358e-3 * window) +
                                 0.011 + 0.478e-3 * hist + 0.64e-3 * window);

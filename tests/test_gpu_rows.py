@@ -315,21 +315,23 @@ def test_rows_past_the_built_in_scratch(dev):
 
 
 @pytest.mark.parametrize("codec,size", [("vq", 8), ("scalar", 3)])
-@pytest.mark.parametrize("T,n,rn,prefill", [(63, 500, 4096, True), (63, 500, 128, False), (63, 30000, 4096, False),
-                                            (16, 500, 4096, False), (32, 500, 16384, True)])
-def test_rows_long_window_chunks(dev, codec, size, T, n, rn, prefill):
+@pytest.mark.parametrize("T,n,rn,prefill,dtype", [(63, 500, 4096, True, torch.bfloat16), (63, 500, 128, False, torch.bfloat16),
+                                                  (63, 30000, 4096, False, torch.bfloat16), (16, 500, 4096, False, torch.bfloat16),
+                                                  (32, 500, 16384, True, torch.bfloat16), (63, 500, 4096, False, torch.float32),
+                                                  (63, 500, 4096, False, torch.float16)])
+def test_rows_long_window_chunks(dev, codec, size, T, n, rn, prefill, dtype):
     """Chunks beside a long exact window: the window's cost counts in the
-    choice between the row and the prefill kernel."""
+    choice between the row and the prefill kernel, where the latter is as exact."""
     strat = _strategy(dev, codec, size)
     st = S.CompressedKVStore(128, 4, device=dev, key_strategy=strat)
-    k = sample_keys(n * 4, seed=n).view(n, 4, 128).bfloat16().to(dev)
+    k = sample_keys(n * 4, seed=n).view(n, 4, 128).to(dtype).to(dev)
     st.append_chunk(k, k)
     q = sample_keys(T * 28, seed=T).view(T, 28, 128).to(dev)
-    kr = sample_keys(rn * 4, seed=rn).view(rn, 4, 128).bfloat16().to(dev)
+    kr = sample_keys(rn * 4, seed=rn).view(rn, 4, 128).to(dtype).to(dev)
     pos = torch.arange(n + rn - T, n + rn, device=dev)
     got, big, ref = (S.compute_hybrid_attention(q, st, kr, kr, 28, query_positions=pos, impl=i) for i in (0, 3, 1))
     assert torch.equal(got, big) == prefill
-    _close(got, ref, (k, kr), f"{codec}{size} T{T} n{n} r{rn}")
+    _close(got, ref, (k, kr), f"{codec}{size} T{T} n{n} r{rn} {dtype}")
 
 
 @pytest.mark.parametrize("size,B,n,T,hq,h,rn,rows", [(8, 512, 16, 3, 32, 8, 0, False), (8, 512, 100, 3, 32, 8, 0, True),
